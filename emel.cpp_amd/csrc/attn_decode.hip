@@ -39,6 +39,7 @@
 #include <cstdlib>
 
 #include "device_common.hpp"
+#include "device_info.hpp"
 #include "emelk.h"
 #include "pool_layout.hpp"
 
@@ -1336,25 +1337,6 @@ struct decode_plan {
   int32_t max_splits = 0;
   uint64_t workspace_bytes = 0;
 };
-
-// Compute units of the current device, cached per device id.  Racing first
-// calls store the same value, so relaxed atomics are enough.
-int32_t device_cu_count() {
-  static std::atomic<int32_t> cached[64];
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-  int32_t cus = cached[dev].load(std::memory_order_relaxed);
-  if (cus == 0) {
-    int c = 0;
-    if (hipDeviceGetAttribute(&c, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-        c <= 0) {
-      c = 256;
-    }
-    cus = c;
-    cached[dev].store(cus, std::memory_order_relaxed);
-  }
-  return cus;
-}
 
 // This is the host plan: the fixed split size, and the bound on the
 // balanced plan the kernels derive on the device for 2 to 64 sequences

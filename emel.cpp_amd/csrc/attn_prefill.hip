@@ -31,6 +31,8 @@
 #include "device_common.hpp"
 #include "emelk.h"
 #include "decode_rows.hpp"
+#include "device_info.hpp"
+#include "prefill_split.hpp"
 #include "pool_layout.hpp"
 
 namespace emelk {
@@ -62,7 +64,25 @@ struct prefill_params {
   int32_t table_stride;
   float c;  // scale * log2(e)
   int32_t bt_shift;  // log2(block_tokens) when a power of two, else -1
+  // Split keys (splits > 1): blockIdx.y is the split; the partials of split s
+  // are part_acc[s][n_seq][n_q][n_head][D], not normalised, and their
+  // (max in raw scores, sum) part_ml[s][n_seq][n_q][n_head][2].
+  int32_t n_seq;
+  int32_t splits;
+  float *part_acc;
+  float *part_ml;
 };
+
+// Split plan of one query tile: its n_tiles key tiles over at most `splits`
+// workgroups, each of at least k_split_min_tiles tiles.  A tile short of
+// twice that keeps one workgroup, which writes the output itself.  The same
+// in the prefill and in the merge kernel.
+constexpr int k_split_min_tiles = 2;
+__host__ __device__ inline int32_t split_tiles(int32_t n_tiles, int32_t splits) {
+  const int32_t most = n_tiles / k_split_min_tiles;
+  const int32_t n = splits < most ? splits : (most < 1 ? 1 : most);
+  return (n_tiles + n - 1) / n;  // tiles per split; 0 without tiles
+}
 
 // Register staging of one key tile.  f16 pools: K as 16-byte row chunks, V
 // as 4 keys x 2 dims.  q8_0 pools: the same items at one byte per value plus
@@ -126,7 +146,7 @@ __device__ __forceinline__ int key_slot16(int k) {
 
 typedef float float4_v __attribute__((ext_vector_type(4)));
 
-template <int D, int G_WG, int RB, int KT, bool Q8, bool M16 = false>
+template <int D, int G_WG, int RB, int KT, bool Q8, bool M16, bool SPLIT>
 __global__ __launch_bounds__(G_WG * RB * k_wave) void prefill_kernel(prefill_params P) {
   constexpr int WAVES = G_WG * RB;
   constexpr int NT = WAVES * k_wave;
@@ -206,7 +226,17 @@ __global__ __launch_bounds__(G_WG * RB * k_wave) void prefill_kernel(prefill_par
   const int total = seq_ok ? q0 + n_q : 0;
   const int wg_row_end = min(n_q, (qt + 1) * RB * ROWS);
   const int key_end = seq_ok ? q0 + wg_row_end : 0;  // exclusive
-  const int n_tiles = (key_end + KT - 1) / KT;
+  const int all_tiles = (key_end + KT - 1) / KT;
+  // key tiles [t_first, n_tiles) of this workgroup
+  int t_first = 0, n_tiles = all_tiles;
+  [[maybe_unused]] bool direct = true;  // the only split of its rows: writes out
+  if constexpr (SPLIT) {
+    const int per = split_tiles(all_tiles, P.splits);
+    t_first = static_cast<int>(blockIdx.y) * per;
+    if (blockIdx.y > 0 && t_first >= all_tiles) return;  // uniform; the merge does not read it
+    n_tiles = min(all_tiles, t_first + per);
+    direct = per >= all_tiles;
+  }
   const int my_row = row0 + (M16 ? c16 : l32);
   const bool row_ok = my_row < n_q;
   const int my_pos = q0 + my_row;
@@ -272,8 +302,9 @@ __global__ __launch_bounds__(G_WG * RB * k_wave) void prefill_kernel(prefill_par
   bool clean;
   const int n_pt = min((n_tiles * KT + P.L.block_tokens - 1) / P.L.block_tokens, k_max_seq_pages);
   {
-    int bad = n_pt * P.L.block_tokens < key_end ? 1 : 0;
-    for (int i = tid; i < n_pt; i += NT) {
+    int bad = n_pt * P.L.block_tokens < min(key_end, n_tiles * KT) ? 1 : 0;
+    const int pt0 = SPLIT ? t_first * KT / P.L.block_tokens : 0;
+    for (int i = pt0 + tid; i < n_pt; i += NT) {
       const uint32_t page = i < P.table_stride ? table[i] : 0xFFFFFFFFu;
       const bool ok = page < static_cast<uint32_t>(P.L.max_blocks);
       s_ptab[i] = ok ? static_cast<uint16_t>(page) : 0xFFFFu;
@@ -360,8 +391,8 @@ __global__ __launch_bounds__(G_WG * RB * k_wave) void prefill_kernel(prefill_par
       __amdgpu_buffer_rsrc_t krs[NS], vrs[NS];
       bool all_valid = true;
       uint32_t pg[NS];
-      if (t == 0) {
-        tile_pages(0, pg);
+      if (t == t_first) {
+        tile_pages(t_first, pg);
       } else {
 #pragma unroll
         for (int j = 0; j < NS; ++j) pg[j] = pg_next[j];
@@ -974,17 +1005,20 @@ __global__ __launch_bounds__(G_WG * RB * k_wave) void prefill_kernel(prefill_par
   };
 
   stage_t R;
-  load_tile(0, R);
-  store_tile(0, 0, R);
+  load_tile(t_first, R);
+  store_tile(t_first & 1, t_first % VR, R);
   __syncthreads();
   float16_v s[NS];
-  // tiles [0, n_int) need no mask
-  const int n_int = clean ? min(n_tiles, min((wg_first_pos + 1) / KT, total / KT)) : 0;
+  // tiles [t_first, n_int) need no mask
+  const int n_int =
+      clean ? max(t_first, min(n_tiles, min((wg_first_pos + 1) / KT, total / KT))) : t_first;
   float4_v s16[2];
   auto step = [&]<bool INTERIOR>(int t) {
     const bool more = t + 1 < n_tiles;
     if (more) load_tile(t + 1, R);
-    if constexpr (M16) {
+    if (SPLIT && row0 >= n_q) {
+      // a row block past the chunk (few rows): it only stages
+    } else if constexpr (M16) {
       qk16(t, s16);
       softmax16.template operator()<INTERIOR>(t, s16);
       pv16(t, s16);
@@ -996,13 +1030,28 @@ __global__ __launch_bounds__(G_WG * RB * k_wave) void prefill_kernel(prefill_par
     if (more) store_tile((t + 1) & 1, (t + 1) % VR, R);
     __syncthreads();
   };
-  for (int t = 0; t < n_int; ++t) step.template operator()<true>(t);
+  for (int t = t_first; t < n_int; ++t) step.template operator()<true>(t);
   for (int t = n_int; t < n_tiles; ++t) step.template operator()<false>(t);
 
-  // normalise by l of each row and write rows < n_q
+  // normalise by l of each row and write rows < n_q (a split writes its
+  // sums as they are, with its rows' m and l)
+  float *dst = P.out;
+  float norm = l > 0.0f ? 1.0f / l : 0.0f;
+  if constexpr (SPLIT) {
+    if (!direct) {
+      const uint64_t rows_all = static_cast<uint64_t>(P.n_seq) * n_q * P.L.n_head;
+      dst = P.part_acc + blockIdx.y * rows_all * D;
+      norm = 1.0f;
+      if (row_ok && (M16 ? g16 == 0 : h == 0)) {
+        float *ml = P.part_ml + (blockIdx.y * rows_all +
+                                 (static_cast<uint64_t>(seq) * n_q + my_row) * P.L.n_head + head) * 2;
+        *reinterpret_cast<float2 *>(ml) = float2{m, l};
+      }
+    }
+  }
   if constexpr (M16) {
     __builtin_amdgcn_wave_barrier();
-    if (g16 == 0) s_row[wave][c16] = l > 0.0f ? 1.0f / l : 0.0f;
+    if (g16 == 0) s_row[wave][c16] = norm;
     __builtin_amdgcn_s_waitcnt(0xc07f);
     __builtin_amdgcn_wave_barrier();
     const float4_t inv = *reinterpret_cast<const float4_t *>(&s_row[wave][4 * g16]);
@@ -1011,14 +1060,14 @@ __global__ __launch_bounds__(G_WG * RB * k_wave) void prefill_kernel(prefill_par
     for (int r = 0; r < 4; ++r) {
       const int row = row0 + 4 * g16 + r;
       if (row >= n_q) continue;
-      float *op = P.out + ((static_cast<uint64_t>(seq) * n_q + row) * P.L.n_head + head) * D;
+      float *op = dst + ((static_cast<uint64_t>(seq) * n_q + row) * P.L.n_head + head) * D;
 #pragma unroll
       for (int c = 0; c < OT16; ++c) op[16 * c + c16] = o16[c][r] * invs[r];
     }
     return;
   }
   __builtin_amdgcn_wave_barrier();
-  if (h == 0) s_row[wave][l32] = l > 0.0f ? 1.0f / l : 0.0f;
+  if (h == 0) s_row[wave][l32] = norm;
   __builtin_amdgcn_s_waitcnt(0xc07f);
   __builtin_amdgcn_wave_barrier();
 #pragma unroll
@@ -1026,34 +1075,151 @@ __global__ __launch_bounds__(G_WG * RB * k_wave) void prefill_kernel(prefill_par
     const int row = row0 + 8 * (r / 4) + 4 * h + (r % 4);
     if (row >= n_q) continue;
     const float inv = s_row[wave][8 * (r / 4) + 4 * h + (r % 4)];
-    float *op = P.out + ((static_cast<uint64_t>(seq) * n_q + row) * P.L.n_head + head) * D;
+    float *op = dst + ((static_cast<uint64_t>(seq) * n_q + row) * P.L.n_head + head) * D;
 #pragma unroll
     for (int c = 0; c < DCH; ++c) op[32 * c + l32] = o[c][r] * inv;
   }
 }
 
-template <int D, int KT, bool Q8, bool M16 = false>
-bool launch_prefill_kt(const prefill_params &P, int32_t n_seq, hipStream_t st) {
-  // W waves per workgroup: G_WG query heads of one KV group x RB blocks of
-  // 32 query rows, all sharing each staged K/V tile.  head_dim 256 runs 4
-  // waves, one per SIMD, so each has the full register file for its 32 x
-  // 256 O tile and Q^T operand (8 waves at head_dim <= 128).
+// Merges the split partials of the rows whose query tile ran in more than one
+// split: o = sum_s 2^{(m_s - M) c} acc_s / sum_s 2^{(m_s - M) c} l_s.  One
+// thread per four dims of one (sequence, row, head).
+constexpr int k_merge_threads = 256;
+template <int D>
+__global__ __launch_bounds__(k_merge_threads) void prefill_merge_kernel(prefill_params P,
+                                                                         int32_t rows_per_tile,
+                                                                         int32_t key_tile) {
+  constexpr int LPR = D / 4;  // threads of a row
+  const uint64_t rows_all = static_cast<uint64_t>(P.n_seq) * P.n_q * P.L.n_head;
+  const uint64_t row = (static_cast<uint64_t>(blockIdx.x) * k_merge_threads + threadIdx.x) / LPR;
+  if (row >= rows_all) return;
+  const uint32_t d = threadIdx.x % LPR * 4;
+  const uint32_t tok = static_cast<uint32_t>(row / P.L.n_head);  // seq * n_q + r
+  const int32_t seq = static_cast<int32_t>(tok / P.n_q);
+  const int32_t r = static_cast<int32_t>(tok % P.n_q);
+  const int32_t q0 = P.q_start[seq];
+  if (q0 < 0) return;  // zeros, written by the first split
+  const int32_t key_end = q0 + min(P.n_q, (r / rows_per_tile + 1) * rows_per_tile);
+  const int32_t n_tiles = (key_end + key_tile - 1) / key_tile;
+  const int32_t per = split_tiles(n_tiles, P.splits);
+  if (per >= n_tiles) return;  // written by its only split
+  const int32_t n = (n_tiles + per - 1) / per;
+  const float *ml = P.part_ml + row * 2;
+  const float *pa = P.part_acc + row * D + d;
+  // batches of loads issued before any is used, with an online max over them
+  constexpr int CH = 8;
+  float mx = -INFINITY, l = 0.0f;
+  float4_t a = {0.0f, 0.0f, 0.0f, 0.0f};
+  for (int32_t s0 = 0; s0 < n; s0 += CH) {
+    float2 mlv[CH];
+    float4_t av[CH];
+#pragma unroll
+    for (int u = 0; u < CH; ++u) {
+      const uint64_t s = static_cast<uint64_t>(s0 + u < n ? s0 + u : s0);
+      mlv[u] = *reinterpret_cast<const float2 *>(ml + s * rows_all * 2);
+      av[u] = *reinterpret_cast<const float4_t *>(pa + s * rows_all * D);
+    }
+    float cm = mlv[0].x;
+#pragma unroll
+    for (int u = 1; u < CH; ++u) cm = fmaxf(cm, mlv[u].x);  // a repeated split changes no max
+    const float mn = fmaxf(mx, cm);
+    const float ms = mn == -INFINITY ? 0.0f : mn;
+    const float f0 = fast_exp2((mx - ms) * P.c);  // 0 on the first batch
+    l *= f0;
+    a *= f0;
+#pragma unroll
+    for (int u = 0; u < CH; ++u) {
+      const float f = s0 + u < n ? fast_exp2((mlv[u].x - ms) * P.c) : 0.0f;
+      l = fmaf(mlv[u].y, f, l);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) a[e] = fmaf(av[u][e], f, a[e]);
+    }
+    mx = mn;
+  }
+  const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+  *reinterpret_cast<float4_t *>(P.out + row * D + d) =
+      float4_t{a.x * inv, a.y * inv, a.z * inv, a.w * inv};
+}
+
+// The launch of one call: W waves per workgroup, G_WG query heads of one KV
+// group x RB blocks of ROWS query rows, all sharing each staged K/V tile.
+// head_dim 256 runs 4 waves, one per SIMD, so each has the full register file
+// for its 32 x 256 O tile and Q^T operand (8 waves at head_dim <= 128).
+struct prefill_shape {
+  int32_t waves, g_wg, rows_per_tile, key_tile;
+  int64_t workgroups;  // without splits
+};
+prefill_shape shape_of(const pool_layout &L, int32_t n_seq, int32_t n_q) {
+  prefill_shape S;
+  S.waves = L.head_dim > 128 ? 4 : 8;
+  const int32_t group = L.n_head / L.n_head_kv;
+  S.g_wg = group < S.waves ? group : S.waves;
+  S.rows_per_tile = (L.head_dim == 512 ? 16 : 32) * (S.waves / S.g_wg);
+  // head_dim 256: 32-key tiles (64 spill, and q8_0's hi/lo K planes of 64-key
+  // tiles would not fit the LDS).  64-key tiles: two independent score chains
+  // per wave and half the barriers of 32-key tiles (measured 834 vs 802
+  // TFLOP/s at the Llama-3-8B chunk shape).
+  S.key_tile = L.head_dim > 128 ? 32 : 64;
+  S.workgroups = static_cast<int64_t>((n_q + S.rows_per_tile - 1) / S.rows_per_tile) *
+                 (L.n_head / S.g_wg) * n_seq;
+  return S;
+}
+
+uint64_t partial_bytes(const pool_layout &L, int32_t n_seq, int32_t n_q) {  // of one split
+  return static_cast<uint64_t>(n_seq) * n_q * L.n_head * (L.head_dim + 2) * sizeof(float);
+}
+
+// Splits of the keys of a call: the count with the least estimated time.  One
+// workgroup runs per CU, so S splits take ceil(workgroups * S / CUs) rounds of
+// ceil(tiles / S) key tiles, and more than one adds the merge launch and one
+// write and one read of the partials.  Measured on MI355X: a key tile takes a
+// workgroup 1.4 us at head_dim 64, 1.9 at 128 (64 keys each), 2.0 at 256 and
+// 3.2 at 512 (32 keys each), and 2.1 times that on q8_0 pools; a split call's
+// start, partial-sum tail and merge cost 6 us, its partials 4.2 TB/s.
+// Examples (unsplit -> split): 5 rows after 2000 tokens, 32/8 heads of 128,
+// 59 -> 13 us; 512 rows of one sequence after 2048, 78 -> 46 (q8_0 165 -> 70);
+// 8/1 heads of 256, 148 -> 40; 512 rows after none, 23.5 us unsplit against
+// 25.7 in four splits, which the estimate leaves unsplit.
+constexpr uint64_t k_split_max_bytes = 64u << 20;
+int32_t plan_splits(const pool_layout &L, const prefill_shape &S, int32_t n_seq, int32_t n_q,
+                    int64_t max_keys) {
+  if (L.head_dim == 512 && L.kv_type == EMELK_KV_Q8_0) return 1;  // row by row
+  const int64_t tiles = (max_keys + S.key_tile - 1) / S.key_tile;
+  const int64_t cus = device_cu_count();
+  int64_t tile_ns = L.head_dim == 64 ? 1400 : L.head_dim == 128 ? 1900 : L.head_dim == 256 ? 2000 : 3200;
+  if (L.kv_type == EMELK_KV_Q8_0) tile_ns = tile_ns * 21 / 10;
+  const uint64_t one = partial_bytes(L, n_seq, n_q);
+  const int64_t merge_ns = static_cast<int64_t>(one) * 2 / 4200;  // of one split's partials
+  int64_t most = tiles / k_split_min_tiles;
+  most = most < cus ? most : cus;
+  if (static_cast<uint64_t>(most) > k_split_max_bytes / one) {
+    most = static_cast<int64_t>(k_split_max_bytes / one);
+  }
+  int64_t best = 1, best_ns = (S.workgroups + cus - 1) / cus * tiles * tile_ns;
+  for (int64_t n = 2; n <= most; ++n) {
+    const int64_t ns = (S.workgroups * n + cus - 1) / cus * ((tiles + n - 1) / n) * tile_ns + 6000 +
+                       n * merge_ns;
+    if (ns < best_ns) {
+      best_ns = ns;
+      best = n;
+    }
+  }
+  return static_cast<int32_t>(best);
+}
+
+template <int D, int KT, bool Q8, bool M16, bool SPLIT>
+bool launch_prefill_kt(const prefill_params &P, const prefill_shape &S, hipStream_t st) {
   constexpr int W = D > 128 ? 4 : 8;
   static_assert(!M16 || W == 4, "M16 runs 4 waves per workgroup");
-  const int group = P.L.n_head / P.L.n_head_kv;
-  const int g_wg = group < W ? group : W;
-  const int rb = W / g_wg;
-  constexpr int ROWS = M16 ? 16 : 32;
-  const int n_qt = (P.n_q + ROWS * rb - 1) / (ROWS * rb);
-  const dim3 grid(n_qt * (P.L.n_head / g_wg) * n_seq);
+  const dim3 grid(static_cast<uint32_t>(S.workgroups), SPLIT ? P.splits : 1);
   const dim3 block(W * k_wave);
-  switch (g_wg) {
-    case 1: hipLaunchKernelGGL((prefill_kernel<D, 1, W, KT, Q8, M16>), grid, block, 0, st, P); return true;
-    case 2: hipLaunchKernelGGL((prefill_kernel<D, 2, W / 2, KT, Q8, M16>), grid, block, 0, st, P); return true;
-    case 4: hipLaunchKernelGGL((prefill_kernel<D, 4, W / 4, KT, Q8, M16>), grid, block, 0, st, P); return true;
+  switch (S.g_wg) {
+    case 1: hipLaunchKernelGGL((prefill_kernel<D, 1, W, KT, Q8, M16, SPLIT>), grid, block, 0, st, P); return true;
+    case 2: hipLaunchKernelGGL((prefill_kernel<D, 2, W / 2, KT, Q8, M16, SPLIT>), grid, block, 0, st, P); return true;
+    case 4: hipLaunchKernelGGL((prefill_kernel<D, 4, W / 4, KT, Q8, M16, SPLIT>), grid, block, 0, st, P); return true;
     case 8:
       if constexpr (W == 8) {
-        hipLaunchKernelGGL((prefill_kernel<D, 8, 1, KT, Q8, M16>), grid, block, 0, st, P);
+        hipLaunchKernelGGL((prefill_kernel<D, 8, 1, KT, Q8, M16, SPLIT>), grid, block, 0, st, P);
         return true;
       }
       return false;
@@ -1061,29 +1227,46 @@ bool launch_prefill_kt(const prefill_params &P, int32_t n_seq, hipStream_t st) {
   }
 }
 
-// 64-key tiles: two independent score chains per wave and half the
-// barriers of 32-key tiles (measured 834 vs 802 TFLOP/s at the Llama-3-8B
-// chunk shape).
-constexpr int k_key_tile = 64;
+template <int D, bool SPLIT>
+bool launch_prefill(const prefill_params &P, const prefill_shape &S, hipStream_t st) {
+  constexpr int KT = D > 128 ? 32 : 64;
+  constexpr bool M16 = D == 512;
+  if constexpr (!M16) {
+    if (P.L.kv_type == EMELK_KV_Q8_0) return launch_prefill_kt<D, KT, true, M16, SPLIT>(P, S, st);
+  }
+  return launch_prefill_kt<D, KT, false, M16, SPLIT>(P, S, st);
+}
 
 template <int D>
-bool launch_prefill(const prefill_params &P, int32_t n_seq, hipStream_t st) {
-  if (P.L.kv_type == EMELK_KV_Q8_0) return launch_prefill_kt<D, k_key_tile, true>(P, n_seq, st);
-  return launch_prefill_kt<D, k_key_tile, false>(P, n_seq, st);
+bool launch_prefill_d(const prefill_params &P, const prefill_shape &S, hipStream_t st) {
+  if (P.splits == 1) return launch_prefill<D, false>(P, S, st);
+  if (!launch_prefill<D, true>(P, S, st)) return false;
+  const uint64_t threads = static_cast<uint64_t>(P.n_seq) * P.n_q * P.L.n_head * (D / 4);
+  const dim3 grid(static_cast<uint32_t>((threads + k_merge_threads - 1) / k_merge_threads));
+  hipLaunchKernelGGL((prefill_merge_kernel<D>), grid, dim3(k_merge_threads), 0, st, P,
+                     S.rows_per_tile, S.key_tile);
+  return true;
 }
 
 }  // namespace
 }  // namespace emelk
 
-extern "C" emel_error_type emelk_attn_prefill_chunk(const emelk_kv_geometry *g, const void *k_pool,
-                                                    const void *v_pool, int32_t layer,
-                                                    const float *q, float *out, int32_t n_seq,
-                                                    int32_t n_q, const int32_t *q_start,
-                                                    const uint16_t *block_tables,
-                                                    int32_t table_stride, float scale,
-                                                    void *stream) {
-  emelk::pool_layout L;
-  if (emelk::make_pool_layout(g, L) != EMELK_ERR_NONE ||
+namespace emelk {
+
+uint64_t prefill_workspace_bound(const emelk_kv_geometry *g, int64_t max_keys) {
+  pool_layout L;
+  if (make_pool_layout(g, L) != EMELK_ERR_NONE) return 0;
+  // a call of one query tile has the most to gain from splits
+  return plan_splits(L, shape_of(L, 1, 1), 1, 1, max_keys) > 1 ? k_split_max_bytes : 0;
+}
+
+emel_error_type prefill_chunk(const emelk_kv_geometry *g, const void *k_pool, const void *v_pool,
+                              int32_t layer, const float *q, float *out, int32_t n_seq,
+                              int32_t n_q, const int32_t *q_start, const uint16_t *block_tables,
+                              int32_t table_stride, float scale, int64_t max_keys,
+                              void *workspace, uint64_t workspace_bytes, void *stream) {
+  pool_layout L;
+  if (make_pool_layout(g, L) != EMELK_ERR_NONE ||
       k_pool == nullptr || v_pool == nullptr || q == nullptr || out == nullptr ||
       q_start == nullptr || block_tables == nullptr || layer < 0 || layer >= L.n_layer ||
       n_seq <= 0 || n_seq > 65535 || n_q <= 0 || table_stride <= 0 || !(scale > 0.0f) ||
@@ -1097,10 +1280,10 @@ extern "C" emel_error_type emelk_attn_prefill_chunk(const emelk_kv_geometry *g, 
     // O tile and Q^T operand take 384 of its 512 registers, and built that
     // way the kernel spills about 1500 registers per lane (about 350 with
     // wave pairs that split O's columns).
-    return emelk::decode_rows(L, k_pool, v_pool, layer, q, out, n_seq, n_q, q_start,
-                              block_tables, table_stride, scale, static_cast<hipStream_t>(stream));
+    return decode_rows(L, k_pool, v_pool, layer, q, out, n_seq, n_q, q_start, block_tables,
+                       table_stride, scale, static_cast<hipStream_t>(stream));
   }
-  emelk::prefill_params P;
+  prefill_params P;
   P.L = L;
   P.k_pool = static_cast<const uint8_t *>(k_pool);
   P.v_pool = static_cast<const uint8_t *>(v_pool);
@@ -1116,16 +1299,61 @@ extern "C" emel_error_type emelk_attn_prefill_chunk(const emelk_kv_geometry *g, 
   for (int b = 0; b < 16; ++b) {
     if ((1 << b) == L.block_tokens) P.bt_shift = b;
   }
+  const prefill_shape S = shape_of(L, n_seq, n_q);
+  const uint64_t one = partial_bytes(L, n_seq, n_q);
+  int64_t splits = workspace == nullptr ? 1 : plan_splits(L, S, n_seq, n_q, max_keys);
+  if (splits > 1 && splits > static_cast<int64_t>(workspace_bytes / one)) {
+    splits = static_cast<int64_t>(workspace_bytes / one);  // as many as the workspace holds
+  }
+  P.n_seq = n_seq;
+  P.splits = splits < 2 ? 1 : static_cast<int32_t>(splits);
+  P.part_acc = static_cast<float *>(workspace);
+  P.part_ml = P.part_acc + static_cast<uint64_t>(P.splits) * n_seq * n_q * L.n_head * L.head_dim;
   hipStream_t st = static_cast<hipStream_t>(stream);
-  const bool q8 = L.kv_type == EMELK_KV_Q8_0;
-  // head_dim 256: 32-key tiles (64 spill, and q8_0's hi/lo K planes of
-  // 64-key tiles would not fit the LDS)
-  const bool ok = L.head_dim == 512 ? emelk::launch_prefill_kt<512, 32, false, true>(P, n_seq, st)
-                  : L.head_dim == 256
-                      ? (q8 ? emelk::launch_prefill_kt<256, 32, true>(P, n_seq, st)
-                            : emelk::launch_prefill_kt<256, 32, false>(P, n_seq, st))
-                  : L.head_dim == 128 ? emelk::launch_prefill<128>(P, n_seq, st)
-                                      : emelk::launch_prefill<64>(P, n_seq, st);
+  const bool ok = L.head_dim == 512   ? launch_prefill_d<512>(P, S, st)
+                  : L.head_dim == 256 ? launch_prefill_d<256>(P, S, st)
+                  : L.head_dim == 128 ? launch_prefill_d<128>(P, S, st)
+                                      : launch_prefill_d<64>(P, S, st);
   if (!ok) return EMELK_ERR_INVALID_REQUEST;
   return hipGetLastError() == hipSuccess ? EMELK_ERR_NONE : EMELK_ERR_BACKEND;
+}
+
+}  // namespace emelk
+
+extern "C" emel_error_type emelk_attn_prefill_chunk(const emelk_kv_geometry *g, const void *k_pool,
+                                                    const void *v_pool, int32_t layer,
+                                                    const float *q, float *out, int32_t n_seq,
+                                                    int32_t n_q, const int32_t *q_start,
+                                                    const uint16_t *block_tables,
+                                                    int32_t table_stride, float scale,
+                                                    void *stream) {
+  return emelk::prefill_chunk(g, k_pool, v_pool, layer, q, out, n_seq, n_q, q_start, block_tables,
+                              table_stride, scale, 0, nullptr, 0, stream);
+}
+
+extern "C" emel_error_type emelk_attn_prefill_workspace_size(const emelk_kv_geometry *g,
+                                                             int32_t n_seq, int32_t n_q,
+                                                             int32_t table_stride,
+                                                             uint64_t *bytes_out) {
+  emelk::pool_layout L;
+  if (emelk::make_pool_layout(g, L) != EMELK_ERR_NONE || bytes_out == nullptr || n_seq <= 0 ||
+      n_seq > 65535 || n_q <= 0 || table_stride <= 0) {
+    return EMELK_ERR_INVALID_REQUEST;
+  }
+  const int32_t splits = emelk::plan_splits(L, emelk::shape_of(L, n_seq, n_q), n_seq, n_q,
+                                            static_cast<int64_t>(table_stride) * L.block_tokens);
+  *bytes_out = splits > 1 ? static_cast<uint64_t>(splits) * emelk::partial_bytes(L, n_seq, n_q) : 0;
+  return EMELK_ERR_NONE;
+}
+
+extern "C" emel_error_type emelk_attn_prefill_chunk_ws(
+    const emelk_kv_geometry *g, const void *k_pool, const void *v_pool, int32_t layer,
+    const float *q, float *out, int32_t n_seq, int32_t n_q, const int32_t *q_start,
+    const uint16_t *block_tables, int32_t table_stride, float scale, void *workspace,
+    uint64_t workspace_bytes, void *stream) {
+  if (g == nullptr || table_stride <= 0) return EMELK_ERR_INVALID_REQUEST;
+  return emelk::prefill_chunk(g, k_pool, v_pool, layer, q, out, n_seq, n_q, q_start, block_tables,
+                              table_stride, scale,
+                              static_cast<int64_t>(table_stride) * g->block_tokens, workspace,
+                              workspace_bytes, stream);
 }

@@ -10,7 +10,8 @@
 // batch), one block-table export for all of them, one upload, and per layer
 // the fused norm + RoPE + append followed by decode (one token per
 // sequence) or chunked-prefill attention (several).  It is a client of the
-// public entry points only.
+// public entry points, and of the split prefill behind
+// emelk_attn_prefill_chunk_ws, which it tells the step's longest sequence.
 #include <hip/hip_runtime_api.h>
 
 #include <algorithm>
@@ -18,6 +19,7 @@
 #include <new>
 
 #include "emelk.h"
+#include "prefill_split.hpp"
 
 struct emelk_batch_decoder {
   emelk_kv_geometry g{};
@@ -84,6 +86,8 @@ extern "C" emel_error_type emelk_batch_decoder_create(const emelk_kv_geometry *g
   if (emelk_attn_decode_workspace_size(g, max_batch, max_kv_len, &ws) != EMELK_ERR_NONE) {
     return EMELK_ERR_INVALID_REQUEST;
   }
+  // one workspace serves both: a layer call runs either
+  ws = std::max(ws, emelk::prefill_workspace_bound(g, max_kv_len));
   auto *d = new (std::nothrow) emelk_batch_decoder();
   if (d == nullptr) return EMELK_ERR_OUT_OF_MEMORY;
   d->g = *g;
@@ -209,13 +213,14 @@ extern "C" emel_error_type emelk_batch_decoder_layer(emelk_batch_decoder *d, int
       &d->g, kp, vp, layer, q_in, q_roped, k_rows, v_rows, d->n_seq, d->n_tokens, d->d_pos,
       d->d_tables, d->stride, d->rope, q_norm, k_norm, v_rms, rms_epsilon, d->stream);
   if (e != EMELK_ERR_NONE) return e;
+  const int32_t plan_len = d->fixed_plan ? d->max_kv_len : d->step_max_kv;
   if (d->n_tokens == 1) {
-    const int32_t plan_len = d->fixed_plan ? d->max_kv_len : d->step_max_kv;
     return emelk_attn_decode(&d->g, kp, vp, layer, q_roped, out, d->n_seq, d->d_kv_len, plan_len,
                              d->d_tables, d->stride, scale, d->d_ws, d->ws_bytes, d->stream);
   }
-  return emelk_attn_prefill_chunk(&d->g, kp, vp, layer, q_roped, out, d->n_seq, d->n_tokens,
-                                  d->d_pos, d->d_tables, d->stride, scale, d->stream);
+  return emelk::prefill_chunk(&d->g, kp, vp, layer, q_roped, out, d->n_seq, d->n_tokens, d->d_pos,
+                              d->d_tables, d->stride, scale, plan_len, d->d_ws, d->ws_bytes,
+                              d->stream);
 }
 
 extern "C" emel_error_type emelk_batch_decoder_set_fixed_plan(emelk_batch_decoder *d, int32_t on) {

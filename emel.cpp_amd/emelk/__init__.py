@@ -230,6 +230,12 @@ _SIGNATURES = [
     ("emelk_attn_prefill_chunk", ctypes.c_uint32,
      [ctypes.POINTER(Geometry), _P, _P, ctypes.c_int32, _P, _P, ctypes.c_int32, ctypes.c_int32,
       _P, _P, ctypes.c_int32, ctypes.c_float, _P]),
+    ("emelk_attn_prefill_workspace_size", ctypes.c_uint32,
+     [ctypes.POINTER(Geometry), ctypes.c_int32, ctypes.c_int32, ctypes.c_int32,
+      ctypes.POINTER(ctypes.c_uint64)]),
+    ("emelk_attn_prefill_chunk_ws", ctypes.c_uint32,
+     [ctypes.POINTER(Geometry), _P, _P, ctypes.c_int32, _P, _P, ctypes.c_int32, ctypes.c_int32,
+      _P, _P, ctypes.c_int32, ctypes.c_float, _P, ctypes.c_uint64, _P]),
     ("emelk_rope_table_create", ctypes.c_uint32,
      [ctypes.POINTER(RopeParams), ctypes.c_int32, ctypes.c_int32, _P,
       ctypes.POINTER(ctypes.c_void_p)]),
@@ -641,6 +647,35 @@ def decode_contiguous(g, k_pool, v_pool, layer, q, out, kv_lens, max_kv_len, seq
         "emelk_attn_decode_contiguous")
 
 
+_PREFILL_WS = {}
+
+
+def _prefill_workspace(g, n_seq, n_q, table_stride, q, stream):
+    """Scratch for the split keys of one prefill call, or None (unsplit).
+
+    It comes from torch's allocator, on the stream the call runs on, so it is
+    reused only by work ordered after the call.  A call on another stream than
+    torch's current one, one under graph capture (whose replays would outlive
+    the scratch) and one on raw addresses run unsplit."""
+    key = (g.n_head, g.n_head_kv, g.head_dim, g.block_tokens, g.kv_type, n_seq, n_q, table_stride)
+    need = _PREFILL_WS.get(key)
+    if need is None:
+        out = ctypes.c_uint64(0)
+        _check(lib.emelk_attn_prefill_workspace_size(ctypes.byref(g), n_seq, n_q, table_stride,
+                                                     ctypes.byref(out)), "prefill_workspace_size")
+        if len(_PREFILL_WS) >= 4096:  # the sizes alone, of as many call shapes
+            _PREFILL_WS.clear()
+        need = _PREFILL_WS[key] = out.value
+    if need == 0 or not _is_tensor(q):
+        return None
+    import torch
+    if stream is not None and stream != torch.cuda.current_stream().cuda_stream:
+        return None
+    if torch.cuda.is_current_stream_capturing():
+        return None
+    return torch.empty(need, dtype=torch.uint8, device="cuda")
+
+
 def prefill_chunk(g, k_pool, v_pool, layer, q, out, q_start, block_tables, scale, stream=None):
     """q/out: float32 [n_seq, n_q, n_head, head_dim]."""
     _pools(g, k_pool, v_pool)
@@ -651,10 +686,12 @@ def prefill_chunk(g, k_pool, v_pool, layer, q, out, q_start, block_tables, scale
     _rows(out, "out", n_seq, n_q, g.n_head * g.head_dim)
     _need(q_start, "q_start", ("int32",), (n_seq,))
     _tables(block_tables, n_seq)
-    _check(lib.emelk_attn_prefill_chunk(ctypes.byref(g), _ptr(k_pool), _ptr(v_pool), layer,
-                                        _ptr(q), _ptr(out), int(q.shape[0]), int(q.shape[1]),
-                                        _ptr(q_start), _ptr(block_tables),
-                                        int(block_tables.shape[1]), scale, _stream(stream)),
+    stride = int(block_tables.shape[1])
+    ws = _prefill_workspace(g, n_seq, n_q, stride, q, stream)
+    _check(lib.emelk_attn_prefill_chunk_ws(ctypes.byref(g), _ptr(k_pool), _ptr(v_pool), layer,
+                                           _ptr(q), _ptr(out), n_seq, n_q, _ptr(q_start),
+                                           _ptr(block_tables), stride, scale, _ptr(ws),
+                                           0 if ws is None else ws.numel(), _stream(stream)),
            "emelk_attn_prefill_chunk")
 
 

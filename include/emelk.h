@@ -351,6 +351,24 @@ emel_error_type emelk_attn_prefill_chunk(const emelk_kv_geometry *g, const void 
                                          const int32_t *q_start, const uint16_t *block_tables,
                                          int32_t table_stride, float scale, void *stream);
 
+/* The same with a workspace, for calls with fewer query tiles than the GPU
+ * has compute units (a few rows, or one sequence's chunk): the keys are then
+ * split over workgroups, whose partial results a second launch merges.  Same
+ * results as emelk_attn_prefill_chunk up to summation order, and deterministic
+ * for the same inputs.  emelk_attn_prefill_workspace_size gives the bytes one
+ * call can use (0 when it would not split; at most 64 MiB); with a
+ * smaller workspace the call runs with fewer splits, and with NULL with none.
+ * Calls that overlap need a workspace each.  The reference has no counterpart. */
+emel_error_type emelk_attn_prefill_workspace_size(const emelk_kv_geometry *g, int32_t n_seq,
+                                                  int32_t n_q, int32_t table_stride,
+                                                  uint64_t *bytes_out);
+emel_error_type emelk_attn_prefill_chunk_ws(const emelk_kv_geometry *g, const void *k_pool,
+                                            const void *v_pool, int32_t layer, const float *q,
+                                            float *out, int32_t n_seq, int32_t n_q,
+                                            const int32_t *q_start, const uint16_t *block_tables,
+                                            int32_t table_stride, float scale, void *workspace,
+                                            uint64_t workspace_bytes, void *stream);
+
 /* RoPE parameters: the reference's rope_pairing (text/generator/detail.hpp:39-50;
  * normal = {2, 2, 1, 0}, neox = {1, 1, 0, 1}) plus n_rot and the frequency base
  * of apply_rope_pairing (detail.hpp:2905-2936).  Pair p rotates dims
