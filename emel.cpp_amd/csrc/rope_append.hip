@@ -12,12 +12,11 @@
 // 1-ulp v_sqrt_f32), so the results are bit-exact against that arithmetic.  cos/sin come from a
 // table built on the host with the reference's recurrence.
 //
-// Launch: one workgroup of 4 waves per (token, group of 4 rows), where the
-// rows of a token are its n_head q heads, n_head_kv k heads and n_head_kv v
-// heads.  A wave stages its row of head_dim floats in its own slice of LDS,
-// so it needs no workgroup barrier, and requests the row together with the
-// token's position.  This is a few KB per token: latency, not bandwidth,
-// bounds it.
+// Launch: a wave takes up to RW rows of one token, where the rows of a token
+// are its n_head q heads, n_head_kv k heads and n_head_kv v heads.  A row lies
+// over D / 4 lanes, four dims each, in registers; the position, page and table
+// reads are per wave (scalar), the (cos, sin) and weights are read once for
+// all of its rows, and no step synchronises across waves.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -27,7 +26,6 @@
 #include "device_common.hpp"
 #include "emelk.h"
 #include "pool_layout.hpp"
-#include "q8_device.hpp"
 
 #pragma clang fp contract(off)
 
@@ -45,14 +43,7 @@ namespace {
 
 using namespace emelk::dev;
 
-constexpr int k_rows_per_wg = 4;
-// rope_append_rows_kernel: rows per wave, and the launch size (rows) from
-// which it replaces rope_append_kernel
-#ifndef EMELK_ROPE_RPW
-#define EMELK_ROPE_RPW 4
-#endif
-constexpr int k_rows_per_wave = EMELK_ROPE_RPW;
-constexpr int64_t k_rows_kernel_min = 1 << 16;
+constexpr int k_waves = 4;  // waves per workgroup
 constexpr int k_max_dim = 512;
 
 struct rope_append_args {
@@ -79,51 +70,125 @@ struct rope_append_args {
   const float *k_norm;
   int32_t v_rms;
   float eps;
+  int32_t pairing;  // rope_pairs
 };
 
-__global__ __launch_bounds__(k_rows_per_wg *k_wave) void rope_append_kernel(rope_append_args A) {
-  __shared__ __align__(16) float s_row[k_rows_per_wg][k_max_dim];  // float4 reads (q8_0)
-  __shared__ float s_scale[k_rows_per_wg];
+// Which dims a pair has: neighbours, the two halves of the head, or any other
+// pairing (rotated through LDS).
+enum rope_pairs : int32_t { k_pairs_none, k_pairs_adjacent, k_pairs_halves, k_pairs_general };
 
-  const pool_layout &L = A.L;
-  const int32_t D = L.head_dim;
-  const int32_t s = blockIdx.x / A.n_tokens;
-  const int32_t t = blockIdx.x % A.n_tokens;
-  const int32_t wave = threadIdx.x / k_wave;
-  const int32_t lane = threadIdx.x % k_wave;
-  const int32_t row = blockIdx.y * k_rows_per_wg + wave;
-  const int32_t n_rows = L.n_head + 2 * L.n_head_kv;
-  const bool have = row < n_rows;
-  const int32_t kind = row < L.n_head ? 0 : (row < L.n_head + L.n_head_kv ? 1 : 2);
-  const int32_t head = kind == 0 ? row : (kind == 1 ? row - L.n_head : row - L.n_head - L.n_head_kv);
-  const uint64_t tok = static_cast<uint64_t>(s) * A.n_tokens + t;
-  // The row is requested together with the position (two floats per lane
-  // per 128 dims), before the token's validity is known.
-  constexpr int NC = k_max_dim / (2 * k_wave);
-  float2 x[NC];
-  if (have) {
-    const float *src =
-        kind == 0 ? A.q_in + (tok * L.n_head + head) * static_cast<uint64_t>(D)
-                  : (kind == 1 ? A.k_rows : A.v_rows) + (tok * L.n_head_kv + head) * static_cast<uint64_t>(D);
+// fp32 rows and weights may lie at any 4-byte address.
+typedef float float4_u __attribute__((ext_vector_type(4), aligned(4)));
+typedef float float2_u __attribute__((ext_vector_type(2), aligned(4)));
+typedef uint32_t uint2_u __attribute__((ext_vector_type(2), aligned(4)));
+
+// apply_rms_norm_in_place's scale (detail.hpp:1098-1106) of one token's whole
+// v, summed in its order: the wave loads 64 values per coalesced load (8 chunks
+// ahead) and every lane adds the squares one by one, each taken from its lane
+// with readlane.
+__device__ __forceinline__ float v_scale(const float *__restrict__ v, int32_t n, int32_t lane,
+                                         float eps) {
+  constexpr int kC = 8;
+  double ss = 0.0;
+  for (int32_t c0 = 0; c0 < n; c0 += kC * k_wave) {
+    float sq[kC];
 #pragma unroll
-    for (int c = 0; c < NC; ++c) {
-      const int32_t d = 2 * (lane + c * k_wave);
-      if (d < D) x[c] = *reinterpret_cast<const float2 *>(src + d);
+    for (int u = 0; u < kC; ++u) {
+      const int32_t i = c0 + u * k_wave + lane;
+      const float x = i < n ? v[i] : 0.0f;
+      sq[u] = x * x;
+    }
+#pragma unroll
+    for (int u = 0; u < kC; ++u) {
+      const int32_t left = n - (c0 + u * k_wave);
+      if (left <= 0) break;  // uniform
+      const double dq = static_cast<double>(sq[u]);
+      if (left >= k_wave) {  // a full chunk: lane indices known at compile time
+#pragma unroll
+        for (int j = 0; j < k_wave; ++j) {
+          const int lo = __builtin_amdgcn_readlane(static_cast<int>(__builtin_bit_cast(uint64_t, dq)), j);
+          const int hi = __builtin_amdgcn_readlane(static_cast<int>(__builtin_bit_cast(uint64_t, dq) >> 32), j);
+          ss += __builtin_bit_cast(double, (static_cast<uint64_t>(static_cast<uint32_t>(hi)) << 32) |
+                                               static_cast<uint32_t>(lo));
+        }
+      } else {
+        for (int32_t j = 0; j < left; ++j) {
+          ss += static_cast<double>(__builtin_bit_cast(
+              float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, sq[u]), j)));
+        }
+      }
     }
   }
-  const int32_t pos = A.positions[s] + t;
+  const float mean = static_cast<float>(ss / static_cast<double>(n));
+  return 1.0f / sqrtf(mean + eps);
+}
+
+// NI row slots per lane: RW = NI * RPI rows per wave, RPI of them per load
+// instruction.  What bounds it: memory for a prompt chunk, latency for a
+// decode step.  The norm's sum must add a row's squares one after another
+// (the reference's order), so the squares go through LDS to one lane per row:
+// RW rows are summed at once, where one lane per wave summing row after row
+// had made it the whole cost.
+template <int D, int NI>
+__global__ __launch_bounds__(k_waves *k_wave) void rope_append_kernel(rope_append_args A) {
+  constexpr int LPR = D / 4 < k_wave ? D / 4 : k_wave;  // lanes of a row
+  constexpr int RPI = k_wave / LPR;                     // rows per load instruction
+  constexpr int NC = D / 4 / LPR;                       // 4-dim chunks of a row per lane
+  constexpr int RW = NI * RPI;
+  constexpr int LROW = D + 4;   // padded LDS row: one lane per row reads without bank conflicts
+  constexpr int NPL = 4;        // (cos, sin) pairs held per lane
+  static_assert(RW <= k_wave, "one lane per row in the norm's sum");
+  extern __shared__ __align__(16) float s_rows[];  // [k_waves][RW][LROW], where a launch needs it
+
+  const pool_layout &L = A.L;
+  const int32_t wave = __builtin_amdgcn_readfirstlane(static_cast<int32_t>(threadIdx.x / k_wave));
+  const int32_t lane = threadIdx.x % k_wave;
+  const uint32_t n_tok = static_cast<uint32_t>(A.n_tokens);
+  const uint32_t tok = blockIdx.x * k_waves + static_cast<uint32_t>(wave);  // < 2^31 (host check)
+  if (tok >= static_cast<uint32_t>(A.n_seq) * n_tok) return;
+  const uint32_t s = tok / n_tok;
+  const int32_t n_qk = L.n_head + L.n_head_kv;
+  const int32_t n_rows = n_qk + L.n_head_kv;
+  const int32_t row0 = static_cast<int32_t>(blockIdx.y) * RW;
+  const int32_t sub = lane / LPR;
+  const int32_t l = lane % LPR;
+
+  // The rows are requested together with the position, before the token's
+  // validity is known.
+  const float *q_src = A.q_in + static_cast<uint64_t>(tok) * L.n_head * D;
+  const float *k_src = A.k_rows + static_cast<uint64_t>(tok) * L.n_head_kv * D;
+  const float *v_src = A.v_rows + static_cast<uint64_t>(tok) * L.n_head_kv * D;
+  float4_t x[NI][NC];
+#pragma unroll
+  for (int i = 0; i < NI; ++i) {
+    const int32_t row = row0 + i * RPI + sub;
+    const float *src = row < L.n_head ? q_src + row * D
+                       : row < n_qk   ? k_src + (row - L.n_head) * D
+                                      : v_src + (row - n_qk) * D;
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      x[i][c] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+      if (row < n_rows) x[i][c] = *reinterpret_cast<const float4_u *>(src + 4 * (l + c * LPR));
+    }
+  }
+  const int32_t pos = A.positions[s] + static_cast<int32_t>(tok - s * n_tok);
   // An invalid token (no position, outside the rope table, past the table
   // row or on an invalid page) writes nothing, q included.
   if (pos < 0) return;
   if (A.pair_count > 0 && pos >= A.rope_positions) return;
-  // the (cos, sin) of the lane's pairs, requested with the page
-  constexpr int NP = k_max_dim / (2 * k_wave);
-  float2 cs[NP];
-  if (have && kind < 2) {
+  const bool rotates = row0 < n_qk && A.pairing != k_pairs_none;  // uniform
+  // adjacent pairs: those of the lane's dims; halves: the four of the lane's
+  // dims, which both halves share; general: pairs lane, lane + 64, ...
+  float2 cs[NPL];
+  if (rotates) {
+    const float2 *table = A.rope + static_cast<uint64_t>(pos) * A.pair_count;
 #pragma unroll
-    for (int c = 0; c < NP; ++c) {
-      const int32_t pr = lane + c * k_wave;
-      if (pr < A.pair_count) cs[c] = A.rope[static_cast<uint64_t>(pos) * A.pair_count + pr];
+    for (int e = 0; e < NPL; ++e) {
+      const int32_t pr = A.pairing == k_pairs_adjacent ? 2 * (l + e / 2 * LPR) + e % 2
+                         : A.pairing == k_pairs_halves ? 4 * l % (D / 2) + e
+                                                       : lane + e * k_wave;
+      cs[e] = float2{1.0f, 0.0f};
+      if (pr < A.pair_count) cs[e] = table[pr];
     }
   }
   const int32_t lb = pos / L.block_tokens;
@@ -131,324 +196,221 @@ __global__ __launch_bounds__(k_rows_per_wg *k_wave) void rope_append_kernel(rope
   const uint32_t page = A.tables[static_cast<uint64_t>(s) * A.table_stride + lb];
   if (page >= static_cast<uint32_t>(L.max_blocks)) return;
   const int32_t slot = pos % L.block_tokens;
-  if (!have) return;  // uniform per wave; nothing below synchronises across waves
-  // Each wave stages only its own row (and its s_scale), so ordering its
-  // own LDS operations is all the synchronisation needed.
+
+  float *buf = s_rows + wave * (RW * LROW);
+  // Each wave stages only its own rows, so ordering its own LDS operations is
+  // all the synchronisation needed.
   auto wave_sync = []() {
     __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
     __builtin_amdgcn_wave_barrier();
   };
-  float *buf = s_row[wave];
-#pragma unroll
-  for (int c = 0; c < NC; ++c) {
-    const int32_t d = 2 * (lane + c * k_wave);
-    if (d < D) *reinterpret_cast<float2 *>(buf + d) = x[c];
-  }
-  wave_sync();
-
-  // Norm scale, computed by one lane in the reference's summation order.
-  const float *wt = kind == 0 ? A.q_norm : (kind == 1 ? A.k_norm : nullptr);
-  const bool head_norm = kind < 2 && wt != nullptr;
-  const bool v_norm = kind == 2 && A.v_rms != 0;
-  if (lane == 0 && head_norm) {
+  if (row0 < n_qk && (A.q_norm != nullptr || A.k_norm != nullptr)) {  // uniform
     // apply_headwise_rms_norm (detail.hpp:1073-1082)
-    float ss = 0.0f;
-    for (int32_t d = 0; d < D; ++d) ss += buf[d] * buf[d];
-    s_scale[wave] = 1.0f / sqrtf(ss / static_cast<float>(D) + A.eps);
-  }
-  if (v_norm) {  // uniform per wave
-    // apply_rms_norm_in_place (detail.hpp:1098-1106) over the token's whole
-    // v, summed in its order: the wave loads 64 values per coalesced load
-    // (8 chunks ahead) and every lane adds the squares one by one, each
-    // taken from its lane with readlane
-    const float *v = A.v_rows + tok * L.n_head_kv * static_cast<uint64_t>(D);
-    const int32_t n = L.n_head_kv * D;
-    constexpr int kC = 8;
-    double ss = 0.0;
-    for (int32_t c0 = 0; c0 < n; c0 += kC * k_wave) {
-      float sq[kC];
 #pragma unroll
-      for (int u = 0; u < kC; ++u) {
-        const int32_t i = c0 + u * k_wave + lane;
-        const float x = i < n ? v[i] : 0.0f;
-        sq[u] = x * x;
+    for (int i = 0; i < NI; ++i) {
+#pragma unroll
+      for (int c = 0; c < NC; ++c) {
+        *reinterpret_cast<float4_t *>(buf + (i * RPI + sub) * LROW + 4 * (l + c * LPR)) =
+            x[i][c] * x[i][c];
       }
+    }
+    wave_sync();
+    float sc = 1.0f;
+    if (lane < RW) {
+      float ss = 0.0f;
+#pragma unroll 16
+      for (int d = 0; d < D; d += 4) {
+        const float4_t sq = *reinterpret_cast<const float4_t *>(buf + lane * LROW + d);
+        ss += sq.x;
+        ss += sq.y;
+        ss += sq.z;
+        ss += sq.w;
+      }
+      sc = 1.0f / sqrtf(ss / static_cast<float>(D) + A.eps);
+    }
+    float4_t wq[NC], wk[NC];
 #pragma unroll
-      for (int u = 0; u < kC; ++u) {
-        const int32_t left = n - (c0 + u * k_wave);
-        if (left <= 0) break;  // uniform
-        const double dq = static_cast<double>(sq[u]);
-        if (left >= k_wave) {  // a full chunk: lane indices known at compile time
+    for (int c = 0; c < NC; ++c) {
+      if (A.q_norm != nullptr) wq[c] = *reinterpret_cast<const float4_u *>(A.q_norm + 4 * (l + c * LPR));
+      if (A.k_norm != nullptr) wk[c] = *reinterpret_cast<const float4_u *>(A.k_norm + 4 * (l + c * LPR));
+    }
 #pragma unroll
-          for (int j = 0; j < k_wave; ++j) {
-            const int lo = __builtin_amdgcn_readlane(static_cast<int>(__builtin_bit_cast(uint64_t, dq)), j);
-            const int hi = __builtin_amdgcn_readlane(static_cast<int>(__builtin_bit_cast(uint64_t, dq) >> 32), j);
-            ss += __builtin_bit_cast(double, (static_cast<uint64_t>(static_cast<uint32_t>(hi)) << 32) |
-                                                 static_cast<uint32_t>(lo));
+    for (int i = 0; i < NI; ++i) {
+      const int32_t row = row0 + i * RPI + sub;
+      const float rs = __shfl(sc, i * RPI + sub, k_wave);
+#pragma unroll
+      for (int c = 0; c < NC; ++c) {
+        if (row < L.n_head) {
+          if (A.q_norm != nullptr) x[i][c] *= rs * wq[c];
+        } else if (row < n_qk) {
+          if (A.k_norm != nullptr) x[i][c] *= rs * wk[c];
+        }
+      }
+    }
+  }
+  if (A.v_rms != 0 && row0 + RW > n_qk) {  // uniform
+    const float rs = v_scale(v_src, L.n_head_kv * D, lane, A.eps);
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+#pragma unroll
+      for (int c = 0; c < NC; ++c) {
+        if (row0 + i * RPI + sub >= n_qk) x[i][c] *= rs;
+      }
+    }
+  }
+
+  // apply_rope_pairing (detail.hpp:2905-2936); pairs never overlap, so their
+  // order does not matter
+  if (rotates && A.pairing == k_pairs_general) {
+    wave_sync();  // the norm's reads are done
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+#pragma unroll
+      for (int c = 0; c < NC; ++c) {
+        *reinterpret_cast<float4_t *>(buf + (i * RPI + sub) * LROW + 4 * (l + c * LPR)) = x[i][c];
+      }
+    }
+    wave_sync();
+    for (int j = 0; j < RW && row0 + j < n_qk; ++j) {  // uniform
+#pragma unroll
+      for (int e = 0; e < NPL; ++e) {
+        const int32_t pr = lane + e * k_wave;
+        if (pr < A.pair_count) {
+          float *b0 = buf + j * LROW + pr * A.x0_stride;
+          float *b1 = buf + j * LROW + pr * A.x1_stride + A.x1_base;
+          const float x0 = *b0;
+          const float x1 = *b1;
+          *b0 = x0 * cs[e].x - x1 * cs[e].y;
+          *b1 = x0 * cs[e].y + x1 * cs[e].x;
+        }
+      }
+    }
+    wave_sync();
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+#pragma unroll
+      for (int c = 0; c < NC; ++c) {
+        x[i][c] = *reinterpret_cast<const float4_t *>(buf + (i * RPI + sub) * LROW + 4 * (l + c * LPR));
+      }
+    }
+  } else if (rotates && A.pairing == k_pairs_halves) {
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      const bool turn = row0 + i * RPI + sub < n_qk;
+      if constexpr (NC == 2) {  // both halves in the lane
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float x0 = x[i][0][e], x1 = x[i][NC - 1][e];
+          if (turn) {
+            x[i][0][e] = x0 * cs[e].x - x1 * cs[e].y;
+            x[i][NC - 1][e] = x0 * cs[e].y + x1 * cs[e].x;
           }
-        } else {
-          for (int32_t j = 0; j < left; ++j) {
-            ss += static_cast<double>(__builtin_bit_cast(
-                float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, sq[u]), j)));
+        }
+      } else {  // the other half lies LPR / 2 lanes away
+        const bool upper = l >= LPR / 2;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float own = x[i][0][e];
+          const float other = __shfl_xor(own, LPR / 2, k_wave);
+          const float x0 = upper ? other : own, x1 = upper ? own : other;
+          const float y = upper ? x0 * cs[e].y + x1 * cs[e].x : x0 * cs[e].x - x1 * cs[e].y;
+          x[i][0][e] = turn ? y : own;
+        }
+      }
+    }
+  } else if (rotates) {
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      const bool turn = row0 + i * RPI + sub < n_qk;
+#pragma unroll
+      for (int c = 0; c < NC; ++c) {
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          const float x0 = x[i][c][2 * e], x1 = x[i][c][2 * e + 1];
+          if (turn && 2 * (l + c * LPR) + e < A.pair_count) {
+            x[i][c][2 * e] = x0 * cs[2 * c + e].x - x1 * cs[2 * c + e].y;
+            x[i][c][2 * e + 1] = x0 * cs[2 * c + e].y + x1 * cs[2 * c + e].x;
           }
         }
       }
     }
-    const float mean = static_cast<float>(ss / static_cast<double>(n));
-    if (lane == 0) s_scale[wave] = 1.0f / sqrtf(mean + A.eps);
-  }
-  if (head_norm || v_norm) {
-    wave_sync();
-    const float sc = s_scale[wave];
-    if (head_norm) {
-      for (int32_t d = lane; d < D; d += k_wave) buf[d] *= sc * wt[d];
-    } else {
-      for (int32_t d = lane; d < D; d += k_wave) buf[d] *= sc;
-    }
-    wave_sync();
   }
 
-  // apply_rope_pairing (detail.hpp:2905-2936): lane p rotates pairs p,
-  // p + 64, ... (pairs never overlap, so the order does not matter)
-  if (kind < 2 && A.pair_count > 0) {
+  const bool q8 = L.kv_type != EMELK_KV_F16;
 #pragma unroll
-    for (int c = 0; c < NP; ++c) {
-      const int32_t pr = lane + c * k_wave;
-      if (pr >= A.pair_count) break;
-      const int32_t d0 = pr * A.x0_stride;
-      const int32_t d1 = pr * A.x1_stride + A.x1_base;
-      const float x0 = buf[d0];
-      const float x1 = buf[d1];
-      buf[d0] = x0 * cs[c].x - x1 * cs[c].y;
-      buf[d1] = x0 * cs[c].y + x1 * cs[c].x;
-    }
-    wave_sync();
-  }
-
-  if (kind == 0) {
-    float *dst = A.q_out + (tok * L.n_head + head) * static_cast<uint64_t>(D);
+  for (int i = 0; i < NI; ++i) {
+    const int32_t row = row0 + i * RPI + sub;
+    const int32_t kvh = row < n_qk ? row - L.n_head : row - n_qk;
+    uint8_t *region = (row < n_qk ? A.k_pool : A.v_pool) +
+                      L.region_offset(A.layer, static_cast<int32_t>(page), kvh);
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
-      const int32_t d = 2 * (lane + c * k_wave);
-      if (d < D) *reinterpret_cast<float2 *>(dst + d) = *reinterpret_cast<const float2 *>(buf + d);
-    }
-    return;
-  }
-  uint8_t *region = (kind == 1 ? A.k_pool : A.v_pool) +
-                    L.region_offset(A.layer, static_cast<int32_t>(page), head);
-  if (L.kv_type == EMELK_KV_F16) {
-    // store_fp16_rounded_cache (detail.hpp:3050-3055): RNE per value
-    uint32_t *dst = reinterpret_cast<uint32_t *>(region + static_cast<uint64_t>(slot) * D * 2u);
-    for (int32_t j = lane; j < D / 2; j += k_wave) dst[j] = as_u32(pack_half2(buf[2 * j], buf[2 * j + 1]));
-  } else {
-    const int32_t blocks = D / 32;
-    if (lane < blocks) {
-      int8_t qs[32];
-      uint16_t dq;
-      quantize_block32(buf + 32 * lane, qs, dq);
-      uint4_t *dst = reinterpret_cast<uint4_t *>(region + static_cast<uint64_t>(slot) * D +
-                                                 static_cast<uint64_t>(lane) * 32u);
-      dst[0] = __builtin_bit_cast(uint4_t, *reinterpret_cast<int8_t(*)[16]>(qs));
-      dst[1] = __builtin_bit_cast(uint4_t, *reinterpret_cast<int8_t(*)[16]>(qs + 16));
-      reinterpret_cast<uint16_t *>(region + L.scale_plane())[static_cast<uint64_t>(slot) * blocks +
-                                                             lane] = dq;
+      const int32_t d = 4 * (l + c * LPR);
+      const float4_t y = x[i][c];
+      if (row < L.n_head) {
+        *reinterpret_cast<float4_u *>(A.q_out + (static_cast<uint64_t>(tok) * L.n_head + row) * D + d) = y;
+      } else if (!q8 && row < n_rows) {
+        // store_fp16_rounded_cache (detail.hpp:3050-3055): RNE per value
+        *reinterpret_cast<uint2_u *>(region + (static_cast<uint64_t>(slot) * D + d) * 2u) =
+            uint2_u{as_u32(pack_half2(y.x, y.y)), as_u32(pack_half2(y.z, y.w))};
+      }
+      if (q8 && row0 + RW > L.n_head) {  // uniform
+        // quantize_row_q8_0_strided (kernel/detail.hpp:804-824) as
+        // quantize_block32: a block is 8 lanes, which share its amax
+        float amax = 0.0f;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) amax = fmaxf(amax, fabsf(y[e]));
+        amax = fmaxf(amax, dpp<k_dpp_quad_xor1>(amax));
+        amax = fmaxf(amax, dpp<k_dpp_quad_xor2>(amax));
+        amax = fmaxf(amax, dpp<k_dpp_row_half_mirror>(amax));
+        const float dq = amax / 127.0f;
+        const float inv = dq != 0.0f ? 1.0f / dq : 0.0f;
+        uint32_t w = 0;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          int q = static_cast<int>(roundf(y[e] * inv));
+          q = q < -127 ? -127 : (q > 127 ? 127 : q);
+          w |= (static_cast<uint32_t>(q) & 0xFFu) << (8 * e);
+        }
+        if (row >= L.n_head && row < n_rows) {
+          *reinterpret_cast<uint32_t *>(region + static_cast<uint64_t>(slot) * D + d) = w;
+          if (l % 8 == 0) {
+            reinterpret_cast<uint16_t *>(region + L.scale_plane())
+                [static_cast<uint64_t>(slot) * (D / 32) + d / 32] = f32_to_f16_bits(dq);
+          }
+        }
+      }
     }
   }
 }
 
-// Large launches (a prefill chunk): each wave takes RPW consecutive
-// (token, row) pairs, token-major, and requests all of their rows and
-// positions, then all of their pages and (cos, sin), before it stages any
-// row, so a wave keeps RPW rows in flight instead of one.  Every loop over
-// the rows is unrolled (the per-row registers stay registers), and the
-// arithmetic per row is that of rope_append_kernel.
-// REG: adjacent pairs (d, d + 1), no norms, f16 pool: a lane's two floats
-// are exactly its pair, so the row never leaves registers.
-template <int D, int RPW, bool REG>
-__global__ __launch_bounds__(k_rows_per_wg *k_wave) void rope_append_rows_kernel(rope_append_args A) {
-  __shared__ __align__(16) float s_row[k_rows_per_wg][D];  // float4 reads (q8_0)
-  __shared__ float s_scale[k_rows_per_wg];
-  constexpr int NC = D / (2 * k_wave) > 0 ? D / (2 * k_wave) : 1;  // float2 per lane per row
-  const pool_layout &L = A.L;
-  const int32_t wave = __builtin_amdgcn_readfirstlane(static_cast<int32_t>(threadIdx.x / k_wave));
-  const int32_t lane = threadIdx.x % k_wave;
-  const uint32_t n_rows = static_cast<uint32_t>(L.n_head + 2 * L.n_head_kv);
-  const uint32_t n_tok = static_cast<uint32_t>(A.n_tokens);
-  const uint32_t total = static_cast<uint32_t>(A.n_seq) * n_tok * n_rows;  // < 2^31 (host check)
-  const uint32_t base = (blockIdx.x * k_rows_per_wg + static_cast<uint32_t>(wave)) * RPW;
-  float *buf = s_row[wave];
-  auto wave_sync = []() {
-    __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
-    __builtin_amdgcn_wave_barrier();
-  };
-
-  uint32_t tok[RPW], seq[RPW];
-  int32_t kind[RPW], head[RPW], pos[RPW];
-  uint32_t page[RPW];
-  bool ok[RPW];
-  float2 x[RPW][NC], cs[RPW][NC];
-#pragma unroll
-  for (int i = 0; i < RPW; ++i) {
-    const uint32_t gr = base + i < total ? base + i : total - 1;  // past the end: a valid address
-    tok[i] = gr / n_rows;
-    const int32_t row = static_cast<int32_t>(gr - tok[i] * n_rows);
-    kind[i] = row < L.n_head ? 0 : (row < L.n_head + L.n_head_kv ? 1 : 2);
-    head[i] = kind[i] == 0 ? row : (kind[i] == 1 ? row - L.n_head : row - L.n_head - L.n_head_kv);
-    const float *src = kind[i] == 0
-                           ? A.q_in + (static_cast<uint64_t>(tok[i]) * L.n_head + head[i]) * D
-                           : (kind[i] == 1 ? A.k_rows : A.v_rows) +
-                                 (static_cast<uint64_t>(tok[i]) * L.n_head_kv + head[i]) * D;
-#pragma unroll
-    for (int c = 0; c < NC; ++c) {
-      const int32_t d = 2 * (lane + c * k_wave);
-      if (d < D) x[i][c] = *reinterpret_cast<const float2 *>(src + d);
-    }
-    seq[i] = tok[i] / n_tok;
-    pos[i] = A.positions[seq[i]] + static_cast<int32_t>(tok[i] - seq[i] * n_tok);
+// Row slots per lane: as many as leave the launch k_enough_waves waves (a
+// prompt chunk), one for a decode step, whose latency counts.  Measured on
+// MI355X with 1 / 2 / 4 / 8 slots at most: 8 x 512 tokens of 16/8 heads of 128
+// with q and k norms and halved pairs 38 / 29 / 28 / 42 us (69 with one lane
+// per wave summing row after row; 4.2 TB/s at 28); 64 x 512 of 32/8 heads,
+// adjacent pairs, 376 / 330 / 304 / 476 (444 before; 4.9 TB/s), on a q8_0 pool
+// 387 / 340 / 313 / 510 (694 with one thread per 32-value block).  A decode
+// step of 8 tokens takes 4.6 us (5.4 before, q8_0 8.3).  Waves of a workgroup
+// that take one token's next rows instead of the next token's same rows were
+// no faster (29 and 315 us at four slots).
+constexpr int k_max_slots = 4;
+constexpr int64_t k_enough_waves = 4096;
+template <int D, int NI>
+bool launch_rope(const rope_append_args &A, hipStream_t st) {
+  constexpr int LPR = D / 4 < k_wave ? D / 4 : k_wave;
+  constexpr int RW = NI * (k_wave / LPR);
+  const int32_t n_rows = A.L.n_head + 2 * A.L.n_head_kv;
+  const int64_t tokens = static_cast<int64_t>(A.n_seq) * A.n_tokens;
+  const int64_t parts = (n_rows + RW - 1) / RW;
+  if constexpr (NI > 1) {
+    if (tokens * parts < k_enough_waves || RW > n_rows) return launch_rope<D, NI / 2>(A, st);
   }
-#pragma unroll
-  for (int i = 0; i < RPW; ++i) {
-    // An invalid token (no position, outside the rope table, past the table
-    // row or on an invalid page) writes nothing, q included.
-    bool v = base + i < total && pos[i] >= 0 &&
-             (A.pair_count == 0 || pos[i] < A.rope_positions);
-    const int32_t lb = v ? pos[i] / L.block_tokens : 0;
-    v = v && lb < A.table_stride;
-    page[i] = v ? static_cast<uint32_t>(A.tables[static_cast<uint64_t>(seq[i]) * A.table_stride + lb])
-                : 0xFFFFFFFFu;
-    ok[i] = page[i] < static_cast<uint32_t>(L.max_blocks);
-#pragma unroll
-    for (int c = 0; c < NC; ++c) {
-      const int32_t pr = lane + c * k_wave;
-      if (v && kind[i] < 2 && pr < A.pair_count) {
-        cs[i][c] = A.rope[static_cast<uint64_t>(pos[i]) * A.pair_count + pr];
-      }
-    }
-  }
-  if constexpr (REG) {
-#pragma unroll
-    for (int i = 0; i < RPW; ++i) {
-      if (!ok[i]) continue;  // uniform
-#pragma unroll
-      for (int c = 0; c < NC; ++c) {
-        const int32_t pr = lane + c * k_wave;  // the lane's pair: dims 2 pr, 2 pr + 1
-        if (2 * pr >= D) continue;
-        float2 y = x[i][c];
-        if (kind[i] < 2 && pr < A.pair_count) {  // apply_rope_pairing, same expressions
-          const float x0 = y.x, x1 = y.y;
-          y.x = x0 * cs[i][c].x - x1 * cs[i][c].y;
-          y.y = x0 * cs[i][c].y + x1 * cs[i][c].x;
-        }
-        if (kind[i] == 0) {
-          *reinterpret_cast<float2 *>(A.q_out + (static_cast<uint64_t>(tok[i]) * L.n_head + head[i]) * D +
-                                      2 * pr) = y;
-        } else {
-          const int32_t slot = pos[i] % L.block_tokens;
-          uint8_t *region = (kind[i] == 1 ? A.k_pool : A.v_pool) +
-                            L.region_offset(A.layer, static_cast<int32_t>(page[i]), head[i]);
-          reinterpret_cast<uint32_t *>(region + static_cast<uint64_t>(slot) * D * 2u)[pr] =
-              as_u32(pack_half2(y.x, y.y));
-        }
-      }
-    }
-    return;
-  }
-#pragma unroll
-  for (int i = 0; i < RPW; ++i) {
-    if (ok[i]) {  // uniform
-#pragma unroll
-      for (int c = 0; c < NC; ++c) {
-        const int32_t d = 2 * (lane + c * k_wave);
-        if (d < D) *reinterpret_cast<float2 *>(buf + d) = x[i][c];
-      }
-      wave_sync();
-      const float *wt = kind[i] == 0 ? A.q_norm : (kind[i] == 1 ? A.k_norm : nullptr);
-      const bool head_norm = kind[i] < 2 && wt != nullptr;
-      const bool v_norm = kind[i] == 2 && A.v_rms != 0;
-      if (lane == 0 && head_norm) {
-        // apply_headwise_rms_norm (detail.hpp:1073-1082)
-        float ss = 0.0f;
-        for (int32_t d = 0; d < D; ++d) ss += buf[d] * buf[d];
-        s_scale[wave] = 1.0f / sqrtf(ss / static_cast<float>(D) + A.eps);
-      }
-      if (v_norm) {
-        // apply_rms_norm_in_place (detail.hpp:1098-1106), in the order of
-        // rope_append_kernel: one fp64 chain over the token's whole v
-        const float *vv = A.v_rows + static_cast<uint64_t>(tok[i]) * L.n_head_kv * D;
-        const int32_t n = L.n_head_kv * D;
-        double ss = 0.0;
-        for (int32_t c0 = 0; c0 < n; c0 += k_wave) {
-          const int32_t j = c0 + lane;
-          const float xv = j < n ? vv[j] : 0.0f;
-          const float sq = xv * xv;
-          const int32_t left = n - c0 < k_wave ? n - c0 : k_wave;
-          for (int32_t l = 0; l < left; ++l) {
-            ss += static_cast<double>(
-                __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, sq), l)));
-          }
-        }
-        const float mean = static_cast<float>(ss / static_cast<double>(n));
-        if (lane == 0) s_scale[wave] = 1.0f / sqrtf(mean + A.eps);
-      }
-      if (head_norm || v_norm) {
-        wave_sync();
-        const float sc = s_scale[wave];
-        if (head_norm) {
-          for (int32_t d = lane; d < D; d += k_wave) buf[d] *= sc * wt[d];
-        } else {
-          for (int32_t d = lane; d < D; d += k_wave) buf[d] *= sc;
-        }
-        wave_sync();
-      }
-      // apply_rope_pairing (detail.hpp:2905-2936)
-      if (kind[i] < 2 && A.pair_count > 0) {
-#pragma unroll
-        for (int c = 0; c < NC; ++c) {
-          const int32_t pr = lane + c * k_wave;
-          if (pr < A.pair_count) {
-            const int32_t d0 = pr * A.x0_stride;
-            const int32_t d1 = pr * A.x1_stride + A.x1_base;
-            const float x0 = buf[d0];
-            const float x1 = buf[d1];
-            buf[d0] = x0 * cs[i][c].x - x1 * cs[i][c].y;
-            buf[d1] = x0 * cs[i][c].y + x1 * cs[i][c].x;
-          }
-        }
-        wave_sync();
-      }
-      if (kind[i] == 0) {
-        float *dst = A.q_out + (static_cast<uint64_t>(tok[i]) * L.n_head + head[i]) * D;
-#pragma unroll
-        for (int c = 0; c < NC; ++c) {
-          const int32_t d = 2 * (lane + c * k_wave);
-          if (d < D) *reinterpret_cast<float2 *>(dst + d) = *reinterpret_cast<const float2 *>(buf + d);
-        }
-      } else {
-        const int32_t slot = pos[i] % L.block_tokens;
-        uint8_t *region = (kind[i] == 1 ? A.k_pool : A.v_pool) +
-                          L.region_offset(A.layer, static_cast<int32_t>(page[i]), head[i]);
-        if (L.kv_type == EMELK_KV_F16) {
-          // store_fp16_rounded_cache (detail.hpp:3050-3055): RNE per value
-          uint32_t *dst = reinterpret_cast<uint32_t *>(region + static_cast<uint64_t>(slot) * D * 2u);
-          for (int32_t j = lane; j < D / 2; j += k_wave) dst[j] = as_u32(pack_half2(buf[2 * j], buf[2 * j + 1]));
-        } else {
-          constexpr int32_t blocks = D / 32;
-          if (lane < blocks) {
-            int8_t qs[32];
-            uint16_t dq;
-            quantize_block32(buf + 32 * lane, qs, dq);
-            uint4_t *dst = reinterpret_cast<uint4_t *>(region + static_cast<uint64_t>(slot) * D +
-                                                       static_cast<uint64_t>(lane) * 32u);
-            dst[0] = __builtin_bit_cast(uint4_t, *reinterpret_cast<int8_t(*)[16]>(qs));
-            dst[1] = __builtin_bit_cast(uint4_t, *reinterpret_cast<int8_t(*)[16]>(qs + 16));
-            reinterpret_cast<uint16_t *>(region + L.scale_plane())[static_cast<uint64_t>(slot) * blocks +
-                                                                   lane] = dq;
-          }
-        }
-      }
-      wave_sync();  // the next row reuses buf
-    }
-  }
+  const bool lds = A.q_norm != nullptr || A.k_norm != nullptr || A.pairing == k_pairs_general;
+  const dim3 grid(static_cast<uint32_t>((tokens + k_waves - 1) / k_waves), static_cast<uint32_t>(parts));
+  hipLaunchKernelGGL((rope_append_kernel<D, NI>), grid, dim3(k_waves * k_wave),
+                     lds ? k_waves * RW * (D + 4) * sizeof(float) : 0, st, A);
+  return hipGetLastError() == hipSuccess;
 }
 
 // Checks a pairing: every pair inside the head and no dim used twice.
@@ -583,35 +545,16 @@ extern "C" emel_error_type emelk_kv_qkv_rope_append(
   A.k_norm = k_norm;
   A.v_rms = v_rms;
   A.eps = rms_epsilon;
-  const int32_t n_rows = L.n_head + 2 * L.n_head_kv;
-  const int64_t rows = static_cast<int64_t>(n_seq) * n_tokens * n_rows;
-  const dim3 block(emelk::k_rows_per_wg * emelk::k_wave);
+  A.pairing = A.pair_count == 0 ? emelk::k_pairs_none
+              : A.x0_stride == 2 && A.x1_stride == 2 && A.x1_base == 1 ? emelk::k_pairs_adjacent
+              : A.x0_stride == 1 && A.x1_stride == 1 && A.x1_base == L.head_dim / 2 &&
+                      A.pair_count == L.head_dim / 2
+                  ? emelk::k_pairs_halves
+                  : emelk::k_pairs_general;
   hipStream_t st = static_cast<hipStream_t>(stream);
-  if (rows >= emelk::k_rows_kernel_min && rows < 0x7FFFFFFF) {
-    constexpr int RPW = emelk::k_rows_per_wave;
-    constexpr int64_t per_wg = emelk::k_rows_per_wg * RPW;
-    const dim3 grid(static_cast<uint32_t>((rows + per_wg - 1) / per_wg));
-    const bool reg = L.kv_type == EMELK_KV_F16 && q_norm == nullptr && k_norm == nullptr &&
-                     v_rms == 0 && A.x0_stride == 2 && A.x1_stride == 2 && A.x1_base == 1;
-    if (reg) {
-      switch (L.head_dim) {
-        case 64: hipLaunchKernelGGL((emelk::rope_append_rows_kernel<64, RPW, true>), grid, block, 0, st, A); break;
-        case 128: hipLaunchKernelGGL((emelk::rope_append_rows_kernel<128, RPW, true>), grid, block, 0, st, A); break;
-        case 256: hipLaunchKernelGGL((emelk::rope_append_rows_kernel<256, RPW, true>), grid, block, 0, st, A); break;
-        default: hipLaunchKernelGGL((emelk::rope_append_rows_kernel<512, RPW, true>), grid, block, 0, st, A); break;
-      }
-    } else {
-      switch (L.head_dim) {
-        case 64: hipLaunchKernelGGL((emelk::rope_append_rows_kernel<64, RPW, false>), grid, block, 0, st, A); break;
-        case 128: hipLaunchKernelGGL((emelk::rope_append_rows_kernel<128, RPW, false>), grid, block, 0, st, A); break;
-        case 256: hipLaunchKernelGGL((emelk::rope_append_rows_kernel<256, RPW, false>), grid, block, 0, st, A); break;
-        default: hipLaunchKernelGGL((emelk::rope_append_rows_kernel<512, RPW, false>), grid, block, 0, st, A); break;
-      }
-    }
-  } else {
-    const dim3 grid(static_cast<uint32_t>(n_seq * n_tokens),
-                    static_cast<uint32_t>((n_rows + emelk::k_rows_per_wg - 1) / emelk::k_rows_per_wg));
-    hipLaunchKernelGGL(emelk::rope_append_kernel, grid, block, 0, st, A);
-  }
-  return hipGetLastError() == hipSuccess ? EMELK_ERR_NONE : EMELK_ERR_BACKEND;
+  const bool ok = L.head_dim == 64    ? emelk::launch_rope<64, emelk::k_max_slots>(A, st)
+                  : L.head_dim == 128 ? emelk::launch_rope<128, emelk::k_max_slots>(A, st)
+                  : L.head_dim == 256 ? emelk::launch_rope<256, emelk::k_max_slots>(A, st)
+                                      : emelk::launch_rope<512, emelk::k_max_slots>(A, st);
+  return ok ? EMELK_ERR_NONE : EMELK_ERR_BACKEND;
 }
