@@ -4,9 +4,11 @@
 // (text/generator/detail.hpp:3153-3230) and its contiguous flash route
 // (kernel/detail.hpp:5238-5291) with one kernel family:
 //
-//   grid = (split, KV-head group, sequence); a workgroup is one wave per KV
-//   head of the group (8 for 8 KV heads), all walking the same pages of one
-//   split of one sequence, so it streams whole pages.  Each wave serves the
+//   grid = (split, KV-head group, sequence); a workgroup has 8 waves (4 at
+//   head_dim 512) over 1 to 8 KV heads, all walking the same pages of one split
+//   of one sequence.  The waves of one KV head take the split's tiles in turn
+//   and merge through LDS: few KV heads, or few sequences, still fill a CU, and
+//   a split leaves one partial per head.  Each wave serves the
 //   G = n_head / n_head_kv query heads of its KV head from the rows it
 //   loads (GQA sharing); the next tile's rows are loaded before the current
 //   tile is used.  q is rounded to fp16 as round_q_for_nonflash does
@@ -36,7 +38,6 @@
 
 #include <cmath>
 #include <atomic>
-#include <cstdlib>
 
 #include "device_common.hpp"
 #include "device_info.hpp"
@@ -67,10 +68,14 @@ constexpr int k_decode_nb = 2;
 // heads instead of 8 ran at 4.44 vs 5.51 TB/s there, and with 3 waves per
 // SIMD (168 VGPRs, one tile set in flight) at 3.06.
 
-// Waves per workgroup = KV heads per workgroup: min(n_head_kv, 8) when it
-// divides n_head_kv, else 1.
-inline int32_t waves_per_block(int32_t n_head_kv) {
-  for (int32_t w = k_max_wpb; w > 1; w >>= 1) {
+// Waves of a workgroup: 8, and 4 at head_dim 512, whose route needs more
+// registers than 8 waves leave each.
+constexpr int k_waves_at(int head_dim) { return head_dim > 256 ? 4 : k_max_wpb; }
+
+// Most KV heads per workgroup (one wave each): the largest power of two up to
+// its waves that divides n_head_kv.
+inline int32_t waves_per_block(int32_t n_head_kv, int32_t head_dim) {
+  for (int32_t w = k_waves_at(head_dim); w > 1; w >>= 1) {
     if (n_head_kv % w == 0) return w;
   }
   return 1;
@@ -105,10 +110,12 @@ struct decode_params {
   // through that sequence's block-table row; null otherwise.
   const int32_t *row_q_start;
   int32_t rows;
-  // Balanced splits (1) or the host plan's fixed split size (0); the host
-  // plan's split size in tiles bounds the balanced one.
+  // Balanced splits (1) or the host plan's fixed split size (0); balanced: the
+  // most splits, and the largest split in tiles.
   int32_t balanced;
-  int32_t host_tiles;
+  int32_t n_seq;
+  int32_t cap;
+  int32_t most_tiles;
   int32_t bt_shift;  // log2(block_tokens) when a power of two, else -1
 };
 
@@ -124,10 +131,11 @@ inline int32_t pow2_shift(int32_t bt) {
 // Balanced split plan of a batch of n_seq <= 64 sequences, the same in every
 // wave that computes it: lane i holds sequence i's length, its split count
 // s_i and the index of its first split (exclusive prefix).  Splits are tb
-// tiles of `tile` tokens, tb = ceil(T / (cap - n_seq)) over the batch's T
-// tiles, clamped to [1, host_tiles]; then sum s_i <= T / tb + n_seq <= cap
-// (or, at tb = host_tiles, <= n_seq * ceil(max tiles / host_tiles) = cap),
-// so every split has a workgroup of the grid and a workspace slot.
+// tiles of `tile` tokens, as few as keep their number within cap (one round of
+// workgroups): tb = ceil(T / (cap - n_seq)) over the batch's T tiles does, as
+// sum s_i <= T / tb + n_seq, and so does most_tiles, at which every sequence is
+// one split (or, past what one split can hold, at most cap / n_seq).  So every
+// split has a workgroup of the grid and a workspace slot.
 // Inclusive prefix sum over the wave by DPP: shifts of 1, 2, 4 and 8 lanes
 // inside each 16-lane row, then lane 15 of a row into the next row and lane
 // 31 into the upper half (row_bcast:15 / row_bcast:31).
@@ -142,15 +150,30 @@ __device__ __forceinline__ int32_t wave_scan_incl(int32_t x) {
 }
 
 __device__ __forceinline__ void balanced_splits(const int32_t *__restrict__ kv_lens, int32_t n_seq,
-                                                int32_t cap, int32_t host_tiles, int32_t tile,
+                                                int32_t cap, int32_t most_tiles, int32_t tile,
                                                 int32_t lane, int32_t &len_i, int32_t &s_i,
                                                 int32_t &excl_i, int32_t &tb) {
   len_i = lane < n_seq ? kv_lens[lane] : 0;
   const int32_t t_i = len_i > 0 ? (len_i + tile - 1) / tile : 0;
   const int32_t incl = wave_scan_incl(t_i);
   const int32_t T = __builtin_amdgcn_readlane(incl, k_wave - 1);
-  tb = cap > n_seq ? (T + (cap - n_seq) - 1) / (cap - n_seq) : host_tiles;
-  tb = tb < 1 ? 1 : (tb > host_tiles ? host_tiles : tb);
+  tb = cap > n_seq ? (T + (cap - n_seq) - 1) / (cap - n_seq) : most_tiles;
+  tb = tb < 1 ? 1 : (tb > most_tiles ? most_tiles : tb);
+  // Fewer tiles per split where they still fit: T / cap, which equal lengths
+  // reach, or what two halvings of the rest up to the bound above find.
+  int32_t lo = T > 0 ? (T + cap - 1) / cap : 1;
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    const int32_t mid = k == 0 ? lo : lo + (tb - lo) / 2;
+    if (lo < tb) {  // uniform
+      const int32_t used = __builtin_amdgcn_readlane(wave_scan_incl((t_i + mid - 1) / mid), k_wave - 1);
+      if (used <= cap) {
+        tb = mid;
+      } else {
+        lo = mid + 1;
+      }
+    }
+  }
   s_i = (t_i + tb - 1) / tb;
   excl_i = wave_scan_incl(s_i) - s_i;
 }
@@ -719,30 +742,41 @@ __device__ __forceinline__ void consume_any(decode_state<D, G, Q8> &S, const til
 //
 // MPV (MQK with UNIFORM): P.V on MFMA as well (consume_tile_mpv); a lane
 // serves one query head per set of 4 (two sets at G = 8).
-template <int D, int G, bool Q8, bool UNIFORM, int WPB, int NB, bool MQK, bool MPV>
-__global__ __launch_bounds__(WPB * k_wave) void decode_kernel(decode_params P) {
+//
+// TS: waves per KV head, which take the split's tiles in turn (token slices)
+// and merge through LDS at the end, so a split leaves one partial per head
+// however many waves walk it.
+template <int D, int G, bool Q8, bool UNIFORM, int WPB, int TS, int NB, bool MQK, bool MPV>
+__global__ __launch_bounds__(WPB * TS * k_wave) void decode_kernel(decode_params P) {
   static_assert(!MPV || (MQK && UNIFORM && G <= 8), "MPV layout");
   constexpr int LPT = D / 16;         // lanes per token row
   constexpr int NGW = k_wave / LPT;   // token groups per wave
   constexpr int TT = 2 * NGW;         // tokens per wave tile
-  constexpr int NT = WPB * k_wave;
+  constexpr int NT = WPB * TS * k_wave;
   constexpr uint32_t ROWB = Q8 ? D : 2 * D;  // bytes of one K/V row in a page
 
   __shared__ uint32_t s_pages[k_max_split_pages];
+  // TS > 1: what each slice found, [head of the workgroup][slice][query head]
+  constexpr int SLOTS = TS > 1 ? WPB * TS * G : 1;
+  __shared__ __align__(16) float s_acc[SLOTS][TS > 1 ? D : 4];
+  __shared__ float2 s_ml[SLOTS];
 
   const int32_t tid = threadIdx.x;
   // the wave index is uniform; readfirstlane lets the compiler keep the
   // head's base pointers in scalar registers
   const int32_t wave = __builtin_amdgcn_readfirstlane(tid / k_wave);
   const int32_t lane = tid % k_wave;
-  const int32_t kvh = blockIdx.y * WPB + wave;
+  const int32_t kvh = blockIdx.y * WPB + wave / TS;
+  const int32_t slice = wave % TS;
   // Start-up in one round trip: the length, q and the split's page-table
   // entries are all requested before any of them is used (the page count
-  // of a split is bounded by tokens_per_split, so the entries are read
-  // before the length is known).
+  // of a split is bounded by its size, so the entries are read before the
+  // length is known).
   // With balanced splits the workgroup first reads every length of the
-  // batch (one more round trip) and takes split w = blockIdx.x + gridDim.x *
-  // blockIdx.z of the balanced plan.  Partial of head h: row slot_base + h *
+  // batch (one more round trip) and takes split w = blockIdx.x of the balanced
+  // plan, whose grid has cap workgroups per head group: idle ones among them
+  // would leave their CUs empty while others hold two (5 sequences of 5000
+  // tokens: 29 us with 35 workgroups per head where 32 run at once).  Partial of head h: row slot_base + h *
   // slot_stride of the workspace.
   int32_t seq = blockIdx.z;
   int32_t split = blockIdx.x;
@@ -751,10 +785,9 @@ __global__ __launch_bounds__(WPB * k_wave) void decode_kernel(decode_params P) {
   uint64_t slot_base;
   uint32_t slot_stride;
   if (P.balanced) {
-    const int32_t w = blockIdx.x + gridDim.x * blockIdx.z;
+    const int32_t w = blockIdx.x;
     int32_t len_i, s_i, excl_i, tb;
-    balanced_splits(P.kv_lens, gridDim.z, gridDim.x * gridDim.z, P.host_tiles, TT, lane, len_i,
-                    s_i, excl_i, tb);
+    balanced_splits(P.kv_lens, P.n_seq, P.cap, P.most_tiles, TT, lane, len_i, s_i, excl_i, tb);
     const uint64_t hit = __builtin_amdgcn_ballot_w64(s_i > 0 && excl_i <= w && w < excl_i + s_i);
     if (hit == 0) return;  // uniform: more workgroups than splits
     seq = __builtin_ctzll(hit);
@@ -795,7 +828,7 @@ __global__ __launch_bounds__(WPB * k_wave) void decode_kernel(decode_params P) {
     }
   }
   constexpr int PPT = (k_max_split_pages + NT - 1) / NT;  // page entries per thread
-  const int32_t max_pages = min(k_max_split_pages, P.tokens_per_split / bt + 2);
+  const int32_t max_pages = min(k_max_split_pages, tps / bt + 2);
   // Null tables: contiguous caches, page = table_row * table_stride + block
   // (no table read between the start and the first tile's loads).
   const bool contiguous = P.tables == nullptr;
@@ -909,10 +942,11 @@ __global__ __launch_bounds__(WPB * k_wave) void decode_kernel(decode_params P) {
   [[maybe_unused]] tile_regs<D, Q8> TN;
   bool has_new = false;
   bool new_ok = false;
-  if (P.new_k != nullptr && len - 1 >= start && len - 1 < end) {  // uniform
+  const bool holds_new = P.new_k != nullptr && len - 1 >= start && len - 1 < end;  // uniform
+  if (holds_new) end = len - 1;
+  if (holds_new && slice == TS - 1) {
     const int32_t p = len - 1;
     has_new = true;
-    end = p;
     const uint32_t page = s_pages[p / bt - first_page];
     new_ok = page != 0xFFFFFFFFu;
     const uint64_t row = (static_cast<uint64_t>(seq) * P.L.n_head_kv + kvh) * D;
@@ -1028,29 +1062,32 @@ __global__ __launch_bounds__(WPB * k_wave) void decode_kernel(decode_params P) {
   // current one is consumed.  (Rotating one set into another with moves
   // would force a wait for the in-flight loads.)  The split's partial last
   // tile, and every tile of a split with an invalid page, run masked after.
-  const int32_t n_full = clean ? (end - start) / TT : 0;
-  int32_t base = start;
+  // Slice s of TS takes tiles s, s + TS, ...
+  constexpr int STEP = TS * TT;
+  const int32_t all_full = clean ? (end - start) / TT : 0;
+  const int32_t n_full = (all_full - slice + TS - 1) / TS;  // this slice's (<= 0: none)
+  int32_t base = start + slice * TT;
   if (n_full > 0) {
     // Loads are unconditional (a load past the last full tile re-reads the
     // last full tile and is discarded): no branch around them, so the
     // compiler's wait counters keep NB - 1 tiles in flight across each
     // consume.  Register set j is only ever touched at unrolled position j.
-    const int32_t last_full = start + (n_full - 1) * TT;
+    const int32_t last_full = base + (n_full - 1) * STEP;
     tile_regs<D, Q8> R[NB];
     bool u0, u1;
 #pragma unroll
     for (int j = 0; j + 1 < NB; ++j) {
-      const int32_t t = start + j * TT;
+      const int32_t t = base + j * STEP;
       load_tile(t <= last_full ? t : last_full, R[j], u0, u1);
     }
     const int32_t n_groups = n_full / NB;
     for (int32_t i = 0; i < n_groups; ++i) {
 #pragma unroll
       for (int j = 0; j < NB; ++j) {
-        const int32_t t = base + (NB - 1) * TT;
+        const int32_t t = base + (NB - 1) * STEP;
         load_tile(t <= last_full ? t : last_full, R[(j + NB - 1) % NB], u0, u1);
         consume_any<D, G, Q8, false, MQK, MPV>(S, R[j], true, true, P.c);
-        base += TT;
+        base += STEP;
       }
     }
     // the remaining n_full % NB tiles are already loaded into R[0..]
@@ -1059,17 +1096,61 @@ __global__ __launch_bounds__(WPB * k_wave) void decode_kernel(decode_params P) {
     for (int j = 0; j + 1 < NB; ++j) {
       if (j < rem) {
         consume_any<D, G, Q8, false, MQK, MPV>(S, R[j], true, true, P.c);
-        base += TT;
+        base += STEP;
       }
     }
   }
-  for (; base < end; base += TT) {
+  for (; base < end; base += STEP) {
     tile_regs<D, Q8> T;
     bool o0, o1;
     load_tile(base, T, o0, o1);
     consume_any<D, G, Q8, true, MQK, MPV>(S, T, o0, o1, P.c);
   }
   if (has_new) consume_any<D, G, Q8, true, MQK, MPV>(S, TN, new_ok && grp == 0, false, P.c);
+
+  // The slices' results (in LDS) as the split's partial, or as the output.
+  auto merge_slices = [&]() {
+    __syncthreads();
+    constexpr int ITEMS = WPB * G * (D / 4);  // four dims of one query head
+    for (int32_t it = tid; it < ITEMS; it += NT) {
+      const int32_t d = it % (D / 4) * 4;
+      const int32_t g = it / (D / 4) % G;
+      const int32_t hl = it / (D / 4) / G;
+      const int32_t first = hl * TS * G + g;
+      float M = -INFINITY;
+#pragma unroll
+      for (int t = 0; t < TS; ++t) M = fmaxf(M, s_ml[first + t * G].x);
+      const float ms = M == -INFINITY ? 0.0f : M;
+      float l = 0.0f;
+      float4_t a = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+      for (int t = 0; t < TS; ++t) {
+        const float2 ml = s_ml[first + t * G];
+        const float f = fast_exp2(ml.x - ms);  // 0 for a slice without tokens
+        l = fmaf(ml.y, f, l);
+        const float4_t v = *reinterpret_cast<const float4_t *>(&s_acc[first + t * G][d]);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) a[e] = fmaf(v[e], f, a[e]);
+      }
+      const int32_t head = (blockIdx.y * WPB + hl) * G + g;
+      if (P.direct_out != nullptr) {
+        const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+        *reinterpret_cast<float4_t *>(
+            P.direct_out + (static_cast<uint64_t>(seq) * P.L.n_head + head) * D + d) =
+            float4_t{a.x * inv, a.y * inv, a.z * inv, a.w * inv};
+      } else {
+        // slot_base is the wave's own KV head's first query head
+        const uint64_t slot = slot_base + static_cast<int64_t>(head - kvh * G) *
+                                              static_cast<int64_t>(slot_stride);
+        *reinterpret_cast<float4_t *>(P.part_acc + slot * D + d) = a;
+        if (d == 0) {
+          P.part_ml[slot * 2] = M;
+          P.part_ml[slot * 2 + 1] = l;
+        }
+      }
+    }
+  };
+  const int32_t my_slot = wave * G;  // (wave / TS * TS + slice) * G: the wave's rows in s_acc
 
   if constexpr (MPV) {
     // Lane (j, chunk, q) holds, for head set hs, head 4 hs + j's 16 dims of
@@ -1124,6 +1205,18 @@ __global__ __launch_bounds__(WPB * k_wave) void decode_kernel(decode_params P) {
       }
       const bool writer = (quad >> RS) == 0 && head < G;
       const uint64_t row = static_cast<uint64_t>(seq) * P.L.n_head + kvh * G + head;
+      if constexpr (TS > 1) {
+        if (writer) {
+#pragma unroll
+          for (int cc = 0; cc < HELD / 4; ++cc) {
+            *reinterpret_cast<float4_t *>(
+                &s_acc[my_slot + head][mpv_dim<D, Q8>(lane_in_row, first_chunk + cc)]) =
+                float4_t{v[4 * cc], v[4 * cc + 1], v[4 * cc + 2], v[4 * cc + 3]};
+          }
+          if (lane_in_row == 0) s_ml[my_slot + head] = float2{M, l};
+        }
+        continue;
+      }
       if (P.direct_out != nullptr) {
         if (writer) {
           const float inv = l > 0.0f ? 1.0f / l : 0.0f;
@@ -1151,6 +1244,7 @@ __global__ __launch_bounds__(WPB * k_wave) void decode_kernel(decode_params P) {
         P.part_ml[slot * 2 + 1] = l;
       }
     }
+    if constexpr (TS > 1) merge_slices();
     return;
   }
   if constexpr (Q8) {
@@ -1211,6 +1305,23 @@ __global__ __launch_bounds__(WPB * k_wave) void decode_kernel(decode_params P) {
 #pragma unroll
   for (int r = 0; r < RS; ++r) first_chunk += ((grp >> r) & 1) * (NCH >> (r + 1));
   const bool writer = (grp >> RS) == 0;  // one lane group per chunk after the sum rounds
+  if constexpr (TS > 1) {
+    if (writer) {
+#pragma unroll
+      for (int c = 0; c < HELD / 4; ++c) {
+        const int ch = first_chunk + c;
+        *reinterpret_cast<float4_t *>(
+            &s_acc[my_slot + ch / 4][lane_dim<D, Q8>(lane_in_row, 4 * (ch % 4))]) =
+            float4_t{v[4 * c], v[4 * c + 1], v[4 * c + 2], v[4 * c + 3]};
+      }
+    }
+    if (lane == 0) {
+#pragma unroll
+      for (int h = 0; h < G; ++h) s_ml[my_slot + h] = float2{M[h], S.l[h]};
+    }
+    merge_slices();
+    return;
+  }
   if (P.direct_out != nullptr) {  // the only split: o = acc / l
     if (writer) {
 #pragma unroll
@@ -1256,28 +1367,36 @@ __global__ __launch_bounds__(WPB * k_wave) void decode_kernel(decode_params P) {
 //
 // Merges the split partials of one (sequence, head): o = sum_s 2^{m_s-M} acc_s
 // / sum_s 2^{m_s-M} l_s (m in the log2 domain, scale folded in).
-template <int D, int CH, bool BAL>
-__global__ __launch_bounds__(D) void combine_kernel(const float *__restrict__ part_acc,
-                                                     const float *__restrict__ part_ml,
-                                                     const int32_t *__restrict__ kv_lens,
-                                                     int32_t n_head, int32_t max_splits,
-                                                     int32_t tokens_per_split,
-                                                     float *__restrict__ out, int32_t n_seq,
-                                                     int32_t host_tiles, int32_t tile) {
+// A workgroup per (sequence, head): D / 4 threads hold four dims each of one
+// split, and the workgroup's R such groups take the splits in turn, so every
+// load of up to R * CH splits is issued before any is used; the groups merge
+// through LDS.
+constexpr int k_combine_threads = 256;
+template <int D, bool BAL>
+__global__ __launch_bounds__(k_combine_threads) void combine_kernel(
+    const float *__restrict__ part_acc, const float *__restrict__ part_ml,
+    const int32_t *__restrict__ kv_lens, int32_t n_head, int32_t max_splits,
+    int32_t tokens_per_split, float *__restrict__ out, int32_t n_seq, int32_t cap,
+    int32_t most_tiles, int32_t tile) {
+  constexpr int LPR = D / 4;
+  constexpr int R = k_combine_threads / LPR;
+  constexpr int CH = 4;
+  __shared__ __align__(16) float s_acc[R][D];
+  __shared__ float2 s_ml[R];
   const int32_t row = blockIdx.x;  // seq * n_head + head
   const int32_t seq = row / n_head;
-  const int32_t d = threadIdx.x;
+  const int32_t grp = threadIdx.x / LPR;
+  const int32_t d = threadIdx.x % LPR * 4;
   // split s of this row is workspace row base + s * stride
   int32_t n;
   uint64_t base;
   [[maybe_unused]] uint64_t stride = 1u;
   if constexpr (BAL) {
     int32_t len_i, s_i, excl_i, tb;
-    balanced_splits(kv_lens, n_seq, n_seq * max_splits, host_tiles, tile, d % k_wave, len_i, s_i,
+    balanced_splits(kv_lens, n_seq, cap, most_tiles, tile, threadIdx.x % k_wave, len_i, s_i,
                     excl_i, tb);
     // lengths past max_kv_len (outside the contract) could plan more splits
     // than the grid ran: read only slots the grid has
-    const int32_t cap = n_seq * max_splits;
     const int32_t first = __builtin_amdgcn_readlane(excl_i, seq);
     n = __builtin_amdgcn_readlane(s_i, seq);
     n = first >= cap ? 0 : min(n, cap - first);
@@ -1290,53 +1409,87 @@ __global__ __launch_bounds__(D) void combine_kernel(const float *__restrict__ pa
   }
   const float *ml = part_ml + base * 2;
   const float *pa = part_acc + base * D + d;
-  // chunks of CH splits: every load of a chunk is issued before any is
-  // used (one round trip for up to CH splits), with an online max across
-  // chunks.  CH is 16 when a sequence has at most 16 splits, else 64
-  // (measured: 16 is 3.5% faster at 15 splits, 64 is 4.7% faster at 33).
-  // Issuing the first chunk's loads before the length arrives (bounded by
-  // max_splits, or at clamped slots) measured slower: 176 and 159 vs 183
-  // GB/s at Qwen3-0.6B, since the slots past the split count cost more than
-  // the length's round trip saves.
-
-  float mx = -INFINITY, l = 0.0f, a = 0.0f;
-  for (int32_t s0 = 0; s0 < n; s0 += CH) {
-    float mv[CH], lv[CH], av[CH];
+  float mx = -INFINITY, l = 0.0f;
+  float4_t a = {0.0f, 0.0f, 0.0f, 0.0f};
+  for (int32_t s0 = grp; s0 < n; s0 += R * CH) {
+    float2 mlv[CH];
+    float4_t av[CH];
 #pragma unroll
     for (int u = 0; u < CH; ++u) {
-      const bool in = s0 + u < n;
-      const uint64_t k = BAL ? (s0 + u) * stride : static_cast<uint64_t>(s0 + u);
-      mv[u] = in ? ml[2 * k] : -INFINITY;
-      lv[u] = in ? ml[2 * k + 1] : 0.0f;
-      av[u] = in ? pa[k * D] : 0.0f;
+      const int32_t sp = s0 + u * R;
+      const uint64_t k = static_cast<uint64_t>(sp < n ? sp : s0) * stride;
+      mlv[u] = *reinterpret_cast<const float2 *>(ml + 2 * k);
+      av[u] = *reinterpret_cast<const float4_t *>(pa + k * D);
     }
-    float cm = mv[0];
+    float cm = mlv[0].x;
 #pragma unroll
-    for (int u = 1; u < CH; ++u) cm = fmaxf(cm, mv[u]);
+    for (int u = 1; u < CH; ++u) cm = fmaxf(cm, mlv[u].x);  // a repeated split changes no max
     const float mn = fmaxf(mx, cm);
     const float ms = mn == -INFINITY ? 0.0f : mn;
-    const float r = fast_exp2(mx - ms);  // 0 on the first chunk
+    const float r = fast_exp2(mx - ms);  // 0 on the first batch
     l *= r;
     a *= r;
-    float lc[2] = {0.0f, 0.0f}, ac[2] = {0.0f, 0.0f};
 #pragma unroll
     for (int u = 0; u < CH; ++u) {
-      const float f = fast_exp2(mv[u] - ms);  // 0 for splits past n
-      lc[u & 1] = fmaf(lv[u], f, lc[u & 1]);
-      ac[u & 1] = fmaf(av[u], f, ac[u & 1]);
+      const float f = s0 + u * R < n ? fast_exp2(mlv[u].x - ms) : 0.0f;
+      l = fmaf(mlv[u].y, f, l);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) a[e] = fmaf(av[u][e], f, a[e]);
     }
-    l += lc[0] + lc[1];
-    a += ac[0] + ac[1];
     mx = mn;
   }
-  out[static_cast<uint64_t>(row) * D + d] = l > 0.0f ? a / l : 0.0f;
+  *reinterpret_cast<float4_t *>(&s_acc[grp][d]) = a;
+  if (d == 0) s_ml[grp] = float2{mx, l};
+  __syncthreads();
+  if (grp != 0) return;
+#pragma unroll
+  for (int g = 1; g < R; ++g) mx = fmaxf(mx, s_ml[g].x);
+  const float ms = mx == -INFINITY ? 0.0f : mx;
+  l = 0.0f;
+  a = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+  for (int g = 0; g < R; ++g) {
+    const float2 gml = s_ml[g];
+    const float f = fast_exp2(gml.x - ms);  // 0 for a group without splits
+    const float4_t v = *reinterpret_cast<const float4_t *>(&s_acc[g][d]);
+    l = fmaf(gml.y, f, l);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) a[e] = fmaf(v[e], f, a[e]);
+  }
+  const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+  *reinterpret_cast<float4_t *>(out + static_cast<uint64_t>(row) * D + d) =
+      float4_t{a.x * inv, a.y * inv, a.z * inv, a.w * inv};
 }
 
 struct decode_plan {
   int32_t tokens_per_split = 0;
   int32_t max_splits = 0;
+  int32_t heads = 0;  // KV heads per workgroup
+  bool balanced = false;  // split sizes from the lengths, on the device
+  int32_t cap = 0;        // balanced: the most splits
+  int32_t most_tiles = 0;  // balanced: the largest split
   uint64_t workspace_bytes = 0;
 };
+
+// KV heads per workgroup: as few as leave every sequence eight splits (so that
+// ragged lengths balance), since a workgroup whose waves walk one head leaves
+// 1/8 of the partials that one of eight heads does.  Measured on MI355X with
+// 1 / 2 / 4 / 8 heads per workgroup (us, 32/8 heads of 128, f16): one sequence
+// of 513 tokens 7.8 / 8.5 / - / 9.2, of 4000 10.3 / 11.0 / - / 15.0; ragged, 3
+// of up to 2000 11.2 / 11.2 / 12.8 / 16.6, 8 of 6000 32.5 / 32.0 / 31.7 / 33.6,
+// 16 of 4097 36.7 / 34.4 / 33.8 / 35.0, 48 of 2000 65 / 62 / 53 / 53.  And
+// what a head's waves taking token slices gives where there are few KV heads:
+// 64 sequences of 8192, 8/1 heads of 256, 272 -> 96 (q8_0 389 -> 86), of 512
+// 794 -> 226, against one wave per KV head and workgroup.
+int32_t plan_heads(const pool_layout &L, int32_t n_seq) {
+  const int32_t most = waves_per_block(L.n_head_kv, L.head_dim);
+  int32_t w = 1;
+  while (w < most && static_cast<int64_t>(device_cu_count()) * w <
+                         int64_t{8} * n_seq * L.n_head_kv) {
+    w <<= 1;
+  }
+  return w;
+}
 
 // This is the host plan: the fixed split size, and the bound on the
 // balanced plan the kernels derive on the device for 2 to 64 sequences
@@ -1346,23 +1499,44 @@ struct decode_plan {
 // what one CU holds at this kernel's register budget; more, shorter splits
 // measured slower because every split pays its page-list load and merge),
 // each split a whole number of wave tiles with its page list inside the LDS
-// cache.
+// cache.  A long context of few KV heads takes up to k_split_tiles tiles per
+// split (one for each of a workgroup's waves) before it takes more than
+// k_few_splits splits, whose merge would cost more than the idle CUs: one
+// sequence of 4000 tokens, 8/1 heads of 256: 17.0 us with 250 splits, 11.8
+// with 63.
+constexpr int32_t k_few_splits = 32;
+constexpr int32_t k_split_tiles = 8;
 decode_plan plan_decode(const pool_layout &L, int32_t n_seq, int32_t max_kv_len) {
   decode_plan p;
+  p.heads = plan_heads(L, n_seq);
   const int32_t lpt = L.head_dim / 16;
   const int32_t tile = 2 * (k_wave / lpt);
-  const int32_t wpb = waves_per_block(L.n_head_kv);
-  const int32_t units = n_seq * (L.n_head_kv / wpb);
+  const int32_t units = n_seq * (L.n_head_kv / p.heads);
   const int32_t target = device_cu_count();
   const int32_t tiles = (max_kv_len + tile - 1) / tile;
-  int32_t splits = (target + units - 1) / units;
-  splits = splits < 1 ? 1 : (splits > tiles ? tiles : splits);
+  int32_t per = (tiles + k_few_splits - 1) / k_few_splits;
+  per = per > k_split_tiles ? k_split_tiles : per;
+  const int32_t most = (tiles + per - 1) / per;
+  const bool may_balance = n_seq > 1 && n_seq <= k_wave;
+  // no more workgroups than run at once (ceil only where the balanced plan's
+  // cap keeps them within that): 24 sequences in 264 workgroups took a second
+  // round for the last eight (55 us; 44 in 256)
+  int32_t splits = may_balance ? (target + units - 1) / units : target / units;
+  splits = splits < 1 ? 1 : (splits > most ? most : splits);
   int32_t tps = ((max_kv_len + splits - 1) / splits + tile - 1) / tile * tile;
   const int32_t max_tps = ((k_max_split_pages - 2) * L.block_tokens) / tile * tile;
   if (tps > max_tps) tps = max_tps;
   if (tps < tile) tps = tile;
   p.tokens_per_split = tps;
   p.max_splits = (max_kv_len + tps - 1) / tps;
+  p.balanced = may_balance && p.max_splits > 1;
+  p.cap = n_seq * p.max_splits;
+  p.most_tiles = tps / tile;
+  const int32_t round = target * p.heads / L.n_head_kv;  // splits whose workgroups run at once
+  if (round >= n_seq && max_kv_len <= max_tps) {
+    p.cap = p.cap < round ? p.cap : round;
+    p.most_tiles = tiles;
+  }
   p.workspace_bytes = static_cast<uint64_t>(n_seq) * L.n_head * p.max_splits *
                       static_cast<uint64_t>(L.head_dim + 2) * sizeof(float);
   return p;
@@ -1371,20 +1545,23 @@ decode_plan plan_decode(const pool_layout &L, int32_t n_seq, int32_t max_kv_len)
 template <int D, int G, bool Q8, int WPB>
 void launch_decode_wpb(const decode_params &P, dim3 grid, hipStream_t st) {
   constexpr int NGW = k_wave / (D / 16);
+  constexpr int TS = k_waves_at(D) / WPB;
   if (P.L.block_tokens % NGW == 0) {
     // MFMA scores and P.V (MPV) up to head_dim 256, any group size
-    hipLaunchKernelGGL((decode_kernel<D, G, Q8, true, WPB, k_decode_nb, D <= 256, D <= 256>),
-                       grid, dim3(WPB * k_wave), 0, st, P);
+    hipLaunchKernelGGL((decode_kernel<D, G, Q8, true, WPB, TS, k_decode_nb, D <= 256, D <= 256>),
+                       grid, dim3(WPB * TS * k_wave), 0, st, P);
   } else {
-    hipLaunchKernelGGL((decode_kernel<D, G, Q8, false, WPB, k_decode_nb, Q8 && D <= 256, false>),
-                       grid, dim3(WPB * k_wave), 0, st, P);
+    hipLaunchKernelGGL((decode_kernel<D, G, Q8, false, WPB, TS, k_decode_nb, Q8 && D <= 256, false>),
+                       grid, dim3(WPB * TS * k_wave), 0, st, P);
   }
 }
 
 template <int D, int G, bool Q8>
-void launch_decode(const decode_params &P, dim3 grid, hipStream_t st) {
-  switch (waves_per_block(P.L.n_head_kv)) {
-    case 8: launch_decode_wpb<D, G, Q8, 8>(P, grid, st); break;
+void launch_decode(int32_t heads, const decode_params &P, dim3 grid, hipStream_t st) {
+  switch (heads) {
+    case 8:
+      if constexpr (k_waves_at(D) == 8) launch_decode_wpb<D, G, Q8, 8>(P, grid, st);
+      break;
     case 4: launch_decode_wpb<D, G, Q8, 4>(P, grid, st); break;
     case 2: launch_decode_wpb<D, G, Q8, 2>(P, grid, st); break;
     default: launch_decode_wpb<D, G, Q8, 1>(P, grid, st); break;
@@ -1392,56 +1569,45 @@ void launch_decode(const decode_params &P, dim3 grid, hipStream_t st) {
 }
 
 template <int D, bool Q8>
-bool dispatch_group(int32_t group, const decode_params &P, dim3 grid, hipStream_t st) {
+bool dispatch_group(int32_t group, int32_t heads, const decode_params &P, dim3 grid, hipStream_t st) {
   switch (group) {
-    case 1: launch_decode<D, 1, Q8>(P, grid, st); return true;
-    case 2: launch_decode<D, 2, Q8>(P, grid, st); return true;
-    case 4: launch_decode<D, 4, Q8>(P, grid, st); return true;
-    case 8: launch_decode<D, 8, Q8>(P, grid, st); return true;
+    case 1: launch_decode<D, 1, Q8>(heads, P, grid, st); return true;
+    case 2: launch_decode<D, 2, Q8>(heads, P, grid, st); return true;
+    case 4: launch_decode<D, 4, Q8>(heads, P, grid, st); return true;
+    case 8: launch_decode<D, 8, Q8>(heads, P, grid, st); return true;
     default: return false;
   }
 }
 
 template <bool Q8>
-bool dispatch_dim(int32_t head_dim, int32_t group, const decode_params &P, dim3 grid,
+bool dispatch_dim(int32_t head_dim, int32_t group, int32_t heads, const decode_params &P, dim3 grid,
                   hipStream_t st) {
   switch (head_dim) {
-    case 64: return dispatch_group<64, Q8>(group, P, grid, st);
-    case 128: return dispatch_group<128, Q8>(group, P, grid, st);
-    case 256: return dispatch_group<256, Q8>(group, P, grid, st);
-    case 512: return dispatch_group<512, Q8>(group, P, grid, st);
+    case 64: return dispatch_group<64, Q8>(group, heads, P, grid, st);
+    case 128: return dispatch_group<128, Q8>(group, heads, P, grid, st);
+    case 256: return dispatch_group<256, Q8>(group, heads, P, grid, st);
+    case 512: return dispatch_group<512, Q8>(group, heads, P, grid, st);
     default: return false;
   }
 }
 
-bool dispatch_decode(const pool_layout &L, const decode_params &P, dim3 grid, hipStream_t st) {
+bool dispatch_decode(const pool_layout &L, int32_t heads, const decode_params &P, dim3 grid,
+                     hipStream_t st) {
   const int32_t group = L.n_head / L.n_head_kv;
-  return L.kv_type == EMELK_KV_Q8_0 ? dispatch_dim<true>(L.head_dim, group, P, grid, st)
-                                    : dispatch_dim<false>(L.head_dim, group, P, grid, st);
+  return L.kv_type == EMELK_KV_Q8_0 ? dispatch_dim<true>(L.head_dim, group, heads, P, grid, st)
+                                    : dispatch_dim<false>(L.head_dim, group, heads, P, grid, st);
 }
 
-template <int D, int CH>
-void launch_combine_d(dim3 grid, hipStream_t st, const decode_params &P, const int32_t *kv_lens,
-                      int32_t n_head, int32_t max_splits, int32_t tps, float *out, int32_t n_seq,
-                      int32_t tile) {
+template <int D>
+void launch_combine(dim3 grid, hipStream_t st, const decode_params &P, const int32_t *kv_lens,
+                    int32_t n_head, int32_t max_splits, int32_t tps, float *out, int32_t n_seq,
+                    int32_t tile) {
   if (P.balanced) {
-    hipLaunchKernelGGL((combine_kernel<D, CH, true>), grid, dim3(D), 0, st, P.part_acc, P.part_ml,
-                       kv_lens, n_head, max_splits, tps, out, n_seq, P.host_tiles, tile);
+    hipLaunchKernelGGL((combine_kernel<D, true>), grid, dim3(k_combine_threads), 0, st, P.part_acc,
+                       P.part_ml, kv_lens, n_head, max_splits, tps, out, n_seq, P.cap, P.most_tiles, tile);
   } else {
-    hipLaunchKernelGGL((combine_kernel<D, CH, false>), grid, dim3(D), 0, st, P.part_acc, P.part_ml,
-                       kv_lens, n_head, max_splits, tps, out, n_seq, P.host_tiles, tile);
-  }
-}
-
-template <int CH>
-void launch_combine_ch(int32_t head_dim, dim3 grid, hipStream_t st, const decode_params &P,
-                       const int32_t *kv_lens, int32_t n_head, int32_t max_splits, int32_t tps,
-                       float *out, int32_t n_seq, int32_t tile) {
-  switch (head_dim) {
-    case 64: launch_combine_d<64, CH>(grid, st, P, kv_lens, n_head, max_splits, tps, out, n_seq, tile); break;
-    case 128: launch_combine_d<128, CH>(grid, st, P, kv_lens, n_head, max_splits, tps, out, n_seq, tile); break;
-    case 256: launch_combine_d<256, CH>(grid, st, P, kv_lens, n_head, max_splits, tps, out, n_seq, tile); break;
-    default: launch_combine_d<512, CH>(grid, st, P, kv_lens, n_head, max_splits, tps, out, n_seq, tile); break;
+    hipLaunchKernelGGL((combine_kernel<D, false>), grid, dim3(k_combine_threads), 0, st, P.part_acc,
+                       P.part_ml, kv_lens, n_head, max_splits, tps, out, n_seq, P.cap, P.most_tiles, tile);
   }
 }
 
@@ -1485,10 +1651,13 @@ emel_error_type decode_rows(const pool_layout &L, const void *k_pool, const void
   P.row_q_start = q_start;
   P.rows = n_q;
   P.balanced = 0;
-  P.host_tiles = 0;
+  P.n_seq = 0;
+  P.cap = 0;
+  P.most_tiles = 0;
   P.bt_shift = pow2_shift(L.block_tokens);
-  const dim3 grid(1, L.n_head_kv / waves_per_block(L.n_head_kv), static_cast<uint32_t>(n_rows));
-  if (!dispatch_decode(L, P, grid, st)) return EMELK_ERR_INVALID_REQUEST;
+  const int32_t heads = waves_per_block(L.n_head_kv, L.head_dim);
+  const dim3 grid(1, L.n_head_kv / heads, static_cast<uint32_t>(n_rows));
+  if (!dispatch_decode(L, heads, P, grid, st)) return EMELK_ERR_INVALID_REQUEST;
   return hipGetLastError() == hipSuccess ? EMELK_ERR_NONE : EMELK_ERR_BACKEND;
 }
 
@@ -1511,7 +1680,7 @@ extern "C" emel_error_type emelk_attn_decode_workspace_size(const emelk_kv_geome
     return EMELK_ERR_INVALID_REQUEST;
   }
   const int32_t tile = 2 * (emelk::k_wave / (L.head_dim / 16));
-  const int32_t wpb = emelk::waves_per_block(L.n_head_kv);
+  const int32_t wpb = emelk::waves_per_block(L.n_head_kv, L.head_dim);
   const int32_t target = emelk::device_cu_count();
   const int64_t tiles = (static_cast<int64_t>(max_kv_len) + tile - 1) / tile;
   const int64_t max_tps = ((emelk::k_max_split_pages - 2) * L.block_tokens) / tile * tile;
@@ -1580,26 +1749,27 @@ emel_error_type decode_impl(const emelk_kv_geometry *g, const void *k_pool, cons
   P.rows = 1;
   // balanced splits for a ragged batch: every split about the same size
   const int32_t tile = 2 * (emelk::k_wave / (L.head_dim / 16));
-  P.balanced = plan.max_splits > 1 && n_seq > 1 && n_seq <= emelk::k_wave ? 1 : 0;
-  P.host_tiles = plan.tokens_per_split / tile;
+  P.balanced = plan.balanced ? 1 : 0;
+  P.n_seq = n_seq;
+  P.cap = plan.cap;
+  P.most_tiles = plan.most_tiles;
   P.bt_shift = emelk::pow2_shift(L.block_tokens);
   P.k_wr = static_cast<uint8_t *>(const_cast<void *>(k_pool));
   P.v_wr = static_cast<uint8_t *>(const_cast<void *>(v_pool));
   const uint64_t acc_floats = static_cast<uint64_t>(n_seq) * L.n_head * plan.max_splits * L.head_dim;
   P.part_acc = static_cast<float *>(workspace);
   P.part_ml = P.part_acc + acc_floats;
-  const dim3 grid(plan.max_splits, L.n_head_kv / emelk::waves_per_block(L.n_head_kv), n_seq);
+  const dim3 grid(plan.balanced ? plan.cap : plan.max_splits, L.n_head_kv / plan.heads,
+                  plan.balanced ? 1 : n_seq);
   hipStream_t st = static_cast<hipStream_t>(stream);
-  if (!emelk::dispatch_decode(L, P, grid, st)) return EMELK_ERR_INVALID_REQUEST;
+  if (!emelk::dispatch_decode(L, plan.heads, P, grid, st)) return EMELK_ERR_INVALID_REQUEST;
   if (P.direct_out != nullptr) return hipGetLastError() == hipSuccess ? EMELK_ERR_NONE : EMELK_ERR_BACKEND;
   const dim3 cgrid(n_seq * L.n_head);
-  if (plan.max_splits > 16) {
-    emelk::launch_combine_ch<64>(L.head_dim, cgrid, st, P, kv_lens, L.n_head, plan.max_splits,
-                                 plan.tokens_per_split, out, n_seq, tile);
-  } else {
-    emelk::launch_combine_ch<16>(L.head_dim, cgrid, st, P, kv_lens, L.n_head, plan.max_splits,
-                                 plan.tokens_per_split, out, n_seq, tile);
-  }
+  const auto combine = L.head_dim == 64    ? emelk::launch_combine<64>
+                       : L.head_dim == 128 ? emelk::launch_combine<128>
+                       : L.head_dim == 256 ? emelk::launch_combine<256>
+                                           : emelk::launch_combine<512>;
+  combine(cgrid, st, P, kv_lens, L.n_head, plan.max_splits, plan.tokens_per_split, out, n_seq, tile);
   return hipGetLastError() == hipSuccess ? EMELK_ERR_NONE : EMELK_ERR_BACKEND;
 }
 

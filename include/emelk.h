@@ -257,8 +257,8 @@ emel_error_type emelk_kv_copy_blocks(const emelk_kv_geometry *g, void *k_pool, v
  * plan (tokens_per_split, n_splits per sequence) and the exact workspace need
  * of one call with these arguments.  For 2 to 64 sequences the device
  * rebalances the splits over the actual lengths (never more splits than
- * n_seq * n_splits, each at most tokens_per_split tokens), so the summation
- * order of a sequence depends on the batch's lengths; results are
+ * n_seq * n_splits), so the summation order of a sequence depends on the
+ * batch's lengths; results are
  * deterministic for the same inputs.  The reference has no counterpart: its
  * CPU route needs no partials. */
 emel_error_type emelk_attn_decode_workspace_size(const emelk_kv_geometry *g, int32_t n_seq,
