@@ -284,9 +284,9 @@ if not os.path.exists(LIB_PATH):
 # device pointers from torch are valid here; loading libemelk.so first would
 # put a second HIP runtime in the process.
 try:
-    import torch  # noqa: F401
+    import torch
 except ImportError:  # plain C/C++ or numpy callers: the system ROCm runtime is used
-    pass
+    torch = None
 lib = ctypes.CDLL(LIB_PATH)
 for _name, _res, _args in _SIGNATURES:
     _fn = getattr(lib, _name)
@@ -435,7 +435,7 @@ def pool_bytes(g: Geometry) -> int:
 
 
 def _ptr(t):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()
 
 
 # Tensor checks run before every device call: a tensor of the wrong dtype,
@@ -484,17 +484,11 @@ _POOL_BYTES = {}
 
 
 def _pool_bytes_cached(g):
-    key = (g.n_layer, g.n_head, g.n_head_kv, g.head_dim, g.block_tokens, g.max_blocks, g.kv_type)
+    key = bytes(g)  # the geometry's fields
     pb = _POOL_BYTES.get(key)
     if pb is None:
         pb = _POOL_BYTES[key] = pool_bytes(g)
     return pb
-
-
-def _pools(g, k_pool, v_pool):
-    pb = _pool_bytes_cached(g)
-    _need(k_pool, "k_pool", min_bytes=pb)
-    _need(v_pool, "v_pool", min_bytes=pb)
 
 
 def _numel(t):
@@ -504,24 +498,67 @@ def _numel(t):
     return n
 
 
-def _rows(t, name, n_seq, n_tokens, width):
-    """fp32 rows [n_seq][n_tokens][width], given as 3-D or flattened."""
-    _need(t, name, ("float32",))
-    if _is_tensor(t) and _numel(t) != n_seq * n_tokens * width:
-        raise ValueError(f"{name}: {_numel(t)} floats, expected {n_seq}*{n_tokens}*{width}")
+def _current_stream():
+    return torch.cuda.current_stream().cuda_stream
 
 
-def _tables(t, n_seq):
-    _need(t, "block_tables", _I16)
-    if _is_tensor(t) and (t.dim() != 2 or int(t.shape[0]) < n_seq):
-        raise ValueError(f"block_tables: shape {tuple(t.shape)}, expected [>= {n_seq}, stride]")
+if torch is not None and hasattr(torch._C, "_cuda_getCurrentRawStream"):
+    # the handle alone, without the Stream object around it
+    def _current_stream():  # noqa: F811
+        return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
 
 def _stream(stream):
-    if stream is not None:
-        return ctypes.c_void_p(stream)
-    import torch
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    return _current_stream() if stream is None else stream
+
+
+# Argument checks.  A plain torch tensor that meets every condition takes one
+# line of tests (a small call is host work first: an append of a few rows and
+# its attention took 23 us with the conditions one by one); anything else goes
+# through _need, which names what is wrong.
+
+_Tensor = torch.Tensor if torch is not None else None
+_f32 = torch.float32 if torch is not None else None
+_i32t = torch.int32 if torch is not None else None
+_tables_dtypes = (torch.int16, torch.uint16) if torch is not None else ()
+
+
+def _pools(g, k_pool, v_pool):
+    pb = _pool_bytes_cached(g)
+    if not (type(k_pool) is _Tensor and k_pool.is_cuda and k_pool.is_contiguous() and
+            k_pool.nbytes >= pb and type(v_pool) is _Tensor and v_pool.is_cuda and
+            v_pool.is_contiguous() and v_pool.nbytes >= pb):
+        _need(k_pool, "k_pool", min_bytes=pb)
+        _need(v_pool, "v_pool", min_bytes=pb)
+
+
+def _rows(t, name, n_seq, n_tokens, width):
+    """fp32 rows [n_seq][n_tokens][width], given as 3-D or flattened."""
+    if not (type(t) is _Tensor and t.is_cuda and t.dtype is _f32 and t.is_contiguous() and
+            t.numel() == n_seq * n_tokens * width):
+        _need(t, name, ("float32",))
+        if _is_tensor(t) and _numel(t) != n_seq * n_tokens * width:
+            raise ValueError(f"{name}: {_numel(t)} floats, expected {n_seq}*{n_tokens}*{width}")
+
+
+def _ints(t, name, n):
+    """int32 [n]."""
+    if not (type(t) is _Tensor and t.is_cuda and t.dtype is _i32t and t.is_contiguous() and
+            t.dim() == 1 and t.numel() == n):
+        _need(t, name, ("int32",), (n,))
+
+
+def _tables(t, n_seq):
+    if not (type(t) is _Tensor and t.is_cuda and t.dtype in _tables_dtypes and
+            t.is_contiguous() and t.dim() == 2 and t.shape[0] >= n_seq):
+        _need(t, "block_tables", _I16)
+        if _is_tensor(t) and (t.dim() != 2 or int(t.shape[0]) < n_seq):
+            raise ValueError(f"block_tables: shape {tuple(t.shape)}, expected [>= {n_seq}, stride]")
+
+
+def _scratch(t):
+    if not (type(t) is _Tensor and t.is_cuda and t.is_contiguous()):
+        _need(t, "workspace")
 
 
 def _check(e, what):
@@ -536,10 +573,11 @@ def append(g, k_pool, v_pool, layer, k_rows, v_rows, positions, block_tables, st
     _pools(g, k_pool, v_pool)
     _rows(k_rows, "k_rows", n_seq, n_tokens, kvd)
     _rows(v_rows, "v_rows", n_seq, n_tokens, kvd)
-    _need(positions, "positions", ("int32",), (n_seq,))
+    _ints(positions, "positions", n_seq)
     _tables(block_tables, n_seq)
-    _check(lib.emelk_kv_append(ctypes.byref(g), _ptr(k_pool), _ptr(v_pool), layer, _ptr(k_rows),
-                               _ptr(v_rows), n_seq, n_tokens, _ptr(positions), _ptr(block_tables),
+    _check(lib.emelk_kv_append(ctypes.byref(g), k_pool.data_ptr(), v_pool.data_ptr(), layer,
+                               k_rows.data_ptr(), v_rows.data_ptr(), n_seq, n_tokens,
+                               positions.data_ptr(), block_tables.data_ptr(),
                                int(block_tables.shape[1]), _stream(stream)), "emelk_kv_append")
 
 
@@ -547,23 +585,23 @@ def gather(g, k_pool, v_pool, layer, lengths, block_tables, k_out, v_out, out_to
            stream=None):
     n_seq = int(lengths.shape[0])
     _pools(g, k_pool, v_pool)
-    _need(lengths, "lengths", ("int32",), (n_seq,))
+    _ints(lengths, "lengths", n_seq)
     _tables(block_tables, n_seq)
     row = g.n_head_kv * g.head_dim * 2 if g.kv_type == KV_F16 else g.n_head_kv * g.head_dim // 32 * 34
     _need(k_out, "k_out", min_bytes=n_seq * out_tokens * row)
     _need(v_out, "v_out", min_bytes=n_seq * out_tokens * row)
-    _check(lib.emelk_kv_gather(ctypes.byref(g), _ptr(k_pool), _ptr(v_pool), layer,
-                               int(lengths.shape[0]), _ptr(lengths), _ptr(block_tables),
-                               int(block_tables.shape[1]), _ptr(k_out), _ptr(v_out), out_tokens,
-                               _stream(stream)), "emelk_kv_gather")
+    _check(lib.emelk_kv_gather(ctypes.byref(g), k_pool.data_ptr(), v_pool.data_ptr(), layer, n_seq,
+                               lengths.data_ptr(), block_tables.data_ptr(), int(block_tables.shape[1]),
+                               k_out.data_ptr(), v_out.data_ptr(), out_tokens, _stream(stream)),
+           "emelk_kv_gather")
 
 
 def copy_blocks(g, k_pool, v_pool, moves, stream=None):
     """moves: int32 [n, 2] device tensor of (src, dst) page ids."""
     _pools(g, k_pool, v_pool)
     _need(moves, "moves", ("int32",), (None, 2))
-    _check(lib.emelk_kv_copy_blocks(ctypes.byref(g), _ptr(k_pool), _ptr(v_pool), _ptr(moves),
-                                    int(moves.shape[0]), _stream(stream)),
+    _check(lib.emelk_kv_copy_blocks(ctypes.byref(g), k_pool.data_ptr(), v_pool.data_ptr(),
+                                    moves.data_ptr(), int(moves.shape[0]), _stream(stream)),
            "emelk_kv_copy_blocks")
 
 
@@ -582,41 +620,43 @@ def decode_plan(g, n_seq, max_kv_len):
     return tps.value, ns.value, int(b.value)
 
 
-def _decode_args(g, k_pool, v_pool, q, out, kv_lens, block_tables, workspace):
+def _decode_args(g, k_pool, v_pool, q, out, kv_lens, workspace):
     _pools(g, k_pool, v_pool)
     if not _is_tensor(q):
         raise TypeError("q: expected a device tensor (its first dimension is n_seq)")
     n_seq = int(q.shape[0])
     _rows(q, "q", n_seq, g.n_head, g.head_dim)
     _rows(out, "out", n_seq, g.n_head, g.head_dim)
-    _need(kv_lens, "kv_lens", ("int32",), (n_seq,))
-    _tables(block_tables, n_seq)
-    _need(workspace, "workspace")
+    _ints(kv_lens, "kv_lens", n_seq)
+    _scratch(workspace)
+    return n_seq
 
 
 def decode(g, k_pool, v_pool, layer, q, out, kv_lens, max_kv_len, block_tables, scale,
            workspace, stream=None):
-    _decode_args(g, k_pool, v_pool, q, out, kv_lens, block_tables, workspace)
-    _check(lib.emelk_attn_decode(ctypes.byref(g), _ptr(k_pool), _ptr(v_pool), layer, _ptr(q),
-                                 _ptr(out), int(q.shape[0]), _ptr(kv_lens), max_kv_len,
-                                 _ptr(block_tables), int(block_tables.shape[1]), scale,
-                                 _ptr(workspace), workspace.numel() * workspace.element_size(),
-                                 _stream(stream)), "emelk_attn_decode")
+    n_seq = _decode_args(g, k_pool, v_pool, q, out, kv_lens, workspace)
+    _tables(block_tables, n_seq)
+    _check(lib.emelk_attn_decode(ctypes.byref(g), k_pool.data_ptr(), v_pool.data_ptr(), layer,
+                                 q.data_ptr(), out.data_ptr(), n_seq, kv_lens.data_ptr(),
+                                 max_kv_len, block_tables.data_ptr(), int(block_tables.shape[1]),
+                                 scale, workspace.data_ptr(),
+                                 workspace.numel() * workspace.element_size(), _stream(stream)),
+           "emelk_attn_decode")
 
 
 def decode_append(g, k_pool, v_pool, layer, k_rows, v_rows, q, out, kv_lens, max_kv_len,
                   block_tables, scale, workspace, stream=None):
     """Store the token at position kv_lens - 1 (k_rows/v_rows float32
     [n_seq, n_head_kv*head_dim]) and attend over kv_lens tokens, one launch."""
-    _decode_args(g, k_pool, v_pool, q, out, kv_lens, block_tables, workspace)
-    n_seq = int(q.shape[0])
+    n_seq = _decode_args(g, k_pool, v_pool, q, out, kv_lens, workspace)
+    _tables(block_tables, n_seq)
     _rows(k_rows, "k_rows", n_seq, 1, g.n_head_kv * g.head_dim)
     _rows(v_rows, "v_rows", n_seq, 1, g.n_head_kv * g.head_dim)
-    _check(lib.emelk_attn_decode_append(ctypes.byref(g), _ptr(k_pool), _ptr(v_pool), layer,
-                                        _ptr(k_rows), _ptr(v_rows), _ptr(q), _ptr(out),
-                                        int(q.shape[0]), _ptr(kv_lens), max_kv_len,
-                                        _ptr(block_tables), int(block_tables.shape[1]), scale,
-                                        _ptr(workspace),
+    _check(lib.emelk_attn_decode_append(ctypes.byref(g), k_pool.data_ptr(), v_pool.data_ptr(),
+                                        layer, k_rows.data_ptr(), v_rows.data_ptr(), q.data_ptr(),
+                                        out.data_ptr(), n_seq, kv_lens.data_ptr(), max_kv_len,
+                                        block_tables.data_ptr(), int(block_tables.shape[1]), scale,
+                                        workspace.data_ptr(),
                                         workspace.numel() * workspace.element_size(),
                                         _stream(stream)), "emelk_attn_decode_append")
 
@@ -626,24 +666,16 @@ def decode_contiguous(g, k_pool, v_pool, layer, q, out, kv_lens, max_kv_len, seq
     """Decode on contiguous caches (no block table): sequence s holds token t
     at page s * seq_stride_tokens / block_tokens + t / block_tokens.  With
     k_rows/v_rows the token at kv_lens - 1 is stored first."""
-    _pools(g, k_pool, v_pool)
-    if not _is_tensor(q):
-        raise TypeError("q: expected a device tensor (its first dimension is n_seq)")
-    n_seq = int(q.shape[0])
-    _rows(q, "q", n_seq, g.n_head, g.head_dim)
-    _rows(out, "out", n_seq, g.n_head, g.head_dim)
-    _need(kv_lens, "kv_lens", ("int32",), (n_seq,))
-    _need(workspace, "workspace")
+    n_seq = _decode_args(g, k_pool, v_pool, q, out, kv_lens, workspace)
     if (k_rows is None) != (v_rows is None):
         raise ValueError("k_rows and v_rows: both or neither")
     if k_rows is not None:
         _rows(k_rows, "k_rows", n_seq, 1, g.n_head_kv * g.head_dim)
         _rows(v_rows, "v_rows", n_seq, 1, g.n_head_kv * g.head_dim)
     _check(lib.emelk_attn_decode_contiguous(
-        ctypes.byref(g), _ptr(k_pool), _ptr(v_pool), layer,
-        _ptr(k_rows), _ptr(v_rows), _ptr(q), _ptr(out), n_seq, _ptr(kv_lens),
-        max_kv_len, seq_stride_tokens, scale, _ptr(workspace),
-        workspace.numel() * workspace.element_size(), _stream(stream)),
+        ctypes.byref(g), k_pool.data_ptr(), v_pool.data_ptr(), layer, _ptr(k_rows), _ptr(v_rows),
+        q.data_ptr(), out.data_ptr(), n_seq, kv_lens.data_ptr(), max_kv_len, seq_stride_tokens,
+        scale, workspace.data_ptr(), workspace.numel() * workspace.element_size(), _stream(stream)),
         "emelk_attn_decode_contiguous")
 
 
@@ -657,7 +689,7 @@ def _prefill_workspace(g, n_seq, n_q, table_stride, q, stream):
     reused only by work ordered after the call.  A call on another stream than
     torch's current one, one under graph capture (whose replays would outlive
     the scratch) and one on raw addresses run unsplit."""
-    key = (g.n_head, g.n_head_kv, g.head_dim, g.block_tokens, g.kv_type, n_seq, n_q, table_stride)
+    key = (bytes(g), n_seq, n_q, table_stride)
     need = _PREFILL_WS.get(key)
     if need is None:
         out = ctypes.c_uint64(0)
@@ -668,8 +700,7 @@ def _prefill_workspace(g, n_seq, n_q, table_stride, q, stream):
         need = _PREFILL_WS[key] = out.value
     if need == 0 or not _is_tensor(q):
         return None
-    import torch
-    if stream is not None and stream != torch.cuda.current_stream().cuda_stream:
+    if stream is not None and stream != _current_stream():
         return None
     if torch.cuda.is_current_stream_capturing():
         return None
@@ -682,15 +713,17 @@ def prefill_chunk(g, k_pool, v_pool, layer, q, out, q_start, block_tables, scale
     if not _is_tensor(q) or q.dim() < 2:
         raise TypeError("q: expected a device tensor [n_seq, n_q, ...]")
     n_seq, n_q = int(q.shape[0]), int(q.shape[1])
-    _rows(q, "q", n_seq, n_q, g.n_head * g.head_dim)
-    _rows(out, "out", n_seq, n_q, g.n_head * g.head_dim)
-    _need(q_start, "q_start", ("int32",), (n_seq,))
+    width = g.n_head * g.head_dim
+    _rows(q, "q", n_seq, n_q, width)
+    _rows(out, "out", n_seq, n_q, width)
+    _ints(q_start, "q_start", n_seq)
     _tables(block_tables, n_seq)
     stride = int(block_tables.shape[1])
     ws = _prefill_workspace(g, n_seq, n_q, stride, q, stream)
-    _check(lib.emelk_attn_prefill_chunk_ws(ctypes.byref(g), _ptr(k_pool), _ptr(v_pool), layer,
-                                           _ptr(q), _ptr(out), n_seq, n_q, _ptr(q_start),
-                                           _ptr(block_tables), stride, scale, _ptr(ws),
+    _check(lib.emelk_attn_prefill_chunk_ws(ctypes.byref(g), k_pool.data_ptr(), v_pool.data_ptr(),
+                                           layer, q.data_ptr(), out.data_ptr(), n_seq, n_q,
+                                           q_start.data_ptr(), block_tables.data_ptr(), stride,
+                                           scale, _ptr(ws),
                                            0 if ws is None else ws.numel(), _stream(stream)),
            "emelk_attn_prefill_chunk")
 
@@ -723,20 +756,22 @@ def qkv_rope_append(g, k_pool, v_pool, layer, q_in, q_out, k_rows, v_rows, posit
     """q_in/q_out: float32 [n_seq, n_tokens, n_head*head_dim]; k_rows/v_rows:
     float32 [n_seq, n_tokens, n_head_kv*head_dim]; all on the device."""
     n_seq, n_tokens = int(k_rows.shape[0]), int(k_rows.shape[1])
+    hd, kvd = g.n_head * g.head_dim, g.n_head_kv * g.head_dim
     _pools(g, k_pool, v_pool)
-    _rows(q_in, "q_in", n_seq, n_tokens, g.n_head * g.head_dim)
-    _rows(q_out, "q_out", n_seq, n_tokens, g.n_head * g.head_dim)
-    _rows(k_rows, "k_rows", n_seq, n_tokens, g.n_head_kv * g.head_dim)
-    _rows(v_rows, "v_rows", n_seq, n_tokens, g.n_head_kv * g.head_dim)
-    _need(positions, "positions", ("int32",), (n_seq,))
+    _rows(q_in, "q_in", n_seq, n_tokens, hd)
+    _rows(q_out, "q_out", n_seq, n_tokens, hd)
+    _rows(k_rows, "k_rows", n_seq, n_tokens, kvd)
+    _rows(v_rows, "v_rows", n_seq, n_tokens, kvd)
+    _ints(positions, "positions", n_seq)
     _tables(block_tables, n_seq)
     _need(q_norm, "q_norm", ("float32",), (g.head_dim,), optional=True)
     _need(k_norm, "k_norm", ("float32",), (g.head_dim,), optional=True)
     _check(lib.emelk_kv_qkv_rope_append(
-        ctypes.byref(g), _ptr(k_pool), _ptr(v_pool), layer, _ptr(q_in), _ptr(q_out),
-        _ptr(k_rows), _ptr(v_rows), n_seq, n_tokens, _ptr(positions), _ptr(block_tables),
-        int(block_tables.shape[1]), rope.handle, _ptr(q_norm), _ptr(k_norm), int(bool(v_rms)),
-        eps, _stream(stream)), "emelk_kv_qkv_rope_append")
+        ctypes.byref(g), k_pool.data_ptr(), v_pool.data_ptr(), layer, q_in.data_ptr(),
+        q_out.data_ptr(), k_rows.data_ptr(), v_rows.data_ptr(), n_seq, n_tokens,
+        positions.data_ptr(), block_tables.data_ptr(), int(block_tables.shape[1]), rope.handle,
+        _ptr(q_norm), _ptr(k_norm), int(bool(v_rms)), eps, _stream(stream)),
+        "emelk_kv_qkv_rope_append")
 
 
 class KvCache:
