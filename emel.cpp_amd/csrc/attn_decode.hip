@@ -1518,10 +1518,12 @@ decode_plan plan_decode(const pool_layout &L, int32_t n_seq, int32_t max_kv_len)
   per = per > k_split_tiles ? k_split_tiles : per;
   const int32_t most = (tiles + per - 1) / per;
   const bool may_balance = n_seq > 1 && n_seq <= k_wave;
-  // no more workgroups than run at once (ceil only where the balanced plan's
-  // cap keeps them within that): 24 sequences in 264 workgroups took a second
-  // round for the last eight (55 us; 44 in 256)
-  int32_t splits = may_balance ? (target + units - 1) / units : target / units;
+  // No more workgroups than run at once: 24 sequences in 264 took a second
+  // round for the last eight (55 us; 39 in 256).  Rounded up where the balanced
+  // plan's cap keeps them within that, and where one split per sequence would
+  // leave a long sequence of a large batch to a single workgroup.
+  const bool up = may_balance || target / units < 2;
+  int32_t splits = up ? (target + units - 1) / units : target / units;
   splits = splits < 1 ? 1 : (splits > most ? most : splits);
   int32_t tps = ((max_kv_len + splits - 1) / splits + tile - 1) / tile * tile;
   const int32_t max_tps = ((k_max_split_pages - 2) * L.block_tokens) / tile * tile;
