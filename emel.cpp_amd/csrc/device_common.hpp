@@ -140,5 +140,13 @@ __device__ __forceinline__ uint4_t load16(const void *p) {
 __device__ __forceinline__ void store16(void *p, uint4_t v) {
   *reinterpret_cast<uint4_t *>(p) = v;
 }
+// The same hint on stores, for copies as large as what they read: they leave the
+// cache to the loads' side.
+__device__ __forceinline__ void store16_stream(void *p, uint4_t v) {
+  __builtin_nontemporal_store(v, reinterpret_cast<uint4_t *>(p));
+}
+__device__ __forceinline__ void store4_stream(void *p, uint32_t v) {
+  __builtin_nontemporal_store(v, reinterpret_cast<uint32_t *>(p));
+}
 
 }  // namespace emelk::dev

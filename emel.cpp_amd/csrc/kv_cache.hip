@@ -119,11 +119,16 @@ __global__ __launch_bounds__(k_threads) void append_q8_0_kernel(
 // Dense head-major copy of logical tokens [0, lengths[s]) through the block
 // table; positions at or past the length are written as zeros.  A workgroup
 // takes runs of tokens of one (sequence, KV head), so those and the destination
-// are uniform and the index work is 32-bit.  f16: 8 sequences of 500 tokens, 8
-// heads of 128, 11.1 -> 9.8 us, of 4096 55.8 -> 54.6 (4.9 TB/s, a large copy's
-// rate); non-temporal loads would take 17.5 instead of 12.9 us where the pool
-// is still in the cache (8 of 4096, one head of 256).
-constexpr int k_gather_tokens = 32;
+// are uniform and the index work is 32-bit.  The output is as large as what is
+// read and goes elsewhere, so its stores carry the non-temporal hint and leave
+// the cache to the pool; the loads do not, since gathered tokens are often still
+// in the cache.  f16, a layer, one division chain per chunk and plain stores ->
+// now: 8 sequences of 4096 tokens, 8 heads of 128 47.8 -> 42.9 us, of 64 27.2 ->
+// 18.3; 6 ragged ones of up to 12632, one head of 512, 55.3 -> 49.5; 8 of 700,
+// two heads of 256, 6.6 -> 5.5.  Hinted loads with plain stores: 17.5 us where
+// both plain take 12.9 (8 of 4096, one head of 256).  Runs of 32 tokens in place
+// of one row piece per thread were slower at head_dim 512 (57.3 us, plain
+// stores, against 53.7).
 
 // Region base of token tok of the workgroup's sequence (its page, its KV head)
 // and the token's row; false where zeros are written.
@@ -157,11 +162,9 @@ __global__ __launch_bounds__(k_threads) void gather_f16_kernel(
     const uint16_t *__restrict__ tables, int32_t table_stride, uint8_t *__restrict__ k_out,
     uint8_t *__restrict__ v_out, int32_t out_tokens) {
   constexpr int CH = D / 8;                      // 16-byte chunks of a row
-  constexpr int TI = k_threads / CH;             // tokens per pass of the workgroup
-  constexpr int N = k_gather_tokens / TI;
-  static_assert(k_gather_tokens % TI == 0, "whole passes");
+  constexpr int T = k_threads / CH;              // tokens of a run
   const uint32_t c = threadIdx.x % CH;
-  const uint32_t runs = (out_tokens - 1) / k_gather_tokens + 1;
+  const uint32_t runs = (out_tokens - 1) / T + 1;
   const uint64_t units = static_cast<uint64_t>(n_seq) * L.n_head_kv * runs;
   for (uint64_t u = blockIdx.x; u < units; u += gridDim.x) {
     const uint32_t sh = static_cast<uint32_t>(u / runs);  // s * n_head_kv + kvh
@@ -171,29 +174,20 @@ __global__ __launch_bounds__(k_threads) void gather_f16_kernel(
     const uint16_t *table = tables + static_cast<uint64_t>(s) * table_stride;
     const uint64_t head_base = L.region_offset(layer, 0, kvh);
     const uint64_t out0 = static_cast<uint64_t>(sh) * out_tokens;
-    const int32_t t0 = static_cast<int32_t>(u - static_cast<uint64_t>(sh) * runs) * k_gather_tokens +
-                       static_cast<int32_t>(threadIdx.x / CH);
-    uint4_t kv[N], vv[N];
-#pragma unroll
-    for (int i = 0; i < N; ++i) {  // every load before any store
-      const gather_src g = gather_at(L, head_base, table, table_stride, len, t0 + i * TI);
-      kv[i] = uint4_t{0u, 0u, 0u, 0u};
-      vv[i] = kv[i];
-      if (g.ok) {
-        const uint64_t src = g.region + (g.row * D + c * 8u) * 2u;
-        kv[i] = load16(k_pool + src);
-        vv[i] = load16(v_pool + src);
-      }
+    const int32_t tok = static_cast<int32_t>(u - static_cast<uint64_t>(sh) * runs) * T +
+                        static_cast<int32_t>(threadIdx.x / CH);
+    if (tok >= out_tokens) continue;
+    const gather_src g = gather_at(L, head_base, table, table_stride, len, tok);
+    uint4_t kval = {0u, 0u, 0u, 0u};
+    uint4_t vval = kval;
+    if (g.ok) {
+      const uint64_t src = g.region + (g.row * D + c * 8u) * 2u;
+      kval = load16(k_pool + src);
+      vval = load16(v_pool + src);
     }
-#pragma unroll
-    for (int i = 0; i < N; ++i) {
-      const int32_t tok = t0 + i * TI;
-      if (tok < out_tokens) {
-        const uint64_t dst = (out0 + tok) * (2u * D) + c * 16u;
-        store16(k_out + dst, kv[i]);
-        store16(v_out + dst, vv[i]);
-      }
-    }
+    const uint64_t dst = (out0 + tok) * (2u * D) + c * 16u;
+    store16_stream(k_out + dst, kval);
+    store16_stream(v_out + dst, vval);
   }
 }
 
@@ -202,7 +196,9 @@ __global__ __launch_bounds__(k_threads) void gather_f16_kernel(
 // but straddle words of the output, so a run's rows (tokens are contiguous in
 // the output) are put together in LDS and leave as words: 17 two-byte stores
 // per block had cost more than the copy (8 sequences of 4096 tokens, 8 heads of
-// 128: 36.1 -> 29.0 us a layer, 4.9 TB/s; 31.8 without the non-temporal loads).
+// 128: 35.9 -> 20 us a layer, 7.1 TB/s; with plain stores 29.1, or 25.4 where
+// the loads carry the non-temporal hint instead, which costs 29.3 against 24.0
+// where the pool is still in the cache).
 template <int D>
 __global__ __launch_bounds__(k_threads) void gather_q8_0_kernel(
     pool_layout L, const uint8_t *__restrict__ k_pool, const uint8_t *__restrict__ v_pool,
@@ -241,8 +237,9 @@ __global__ __launch_bounds__(k_threads) void gather_q8_0_kernel(
         d[kv][i] = 0u;
         if (g.ok) {
           const uint8_t *region = (kv == 0 ? k_pool : v_pool) + g.region;
-          q[kv][i] = load16_stream(region + g.row * D + c * 16u);
-          d[kv][i] = load2_stream(region + splane + (g.row * (D / 32) + c / 2) * 2u);
+          q[kv][i] = load16(region + g.row * D + c * 16u);
+          d[kv][i] = *reinterpret_cast<const uint16_t *>(region + splane +
+                                                         (g.row * (D / 32) + c / 2) * 2u);
         }
       }
     }
@@ -274,7 +271,7 @@ __global__ __launch_bounds__(k_threads) void gather_q8_0_kernel(
       uint8_t *out = (kv == 0 ? k_out : v_out) + dst;
       if ((reinterpret_cast<uintptr_t>(out) & 3u) == 0) {
         for (int32_t b = threadIdx.x * 4; b < bytes; b += k_threads * 4) {
-          *reinterpret_cast<uint32_t *>(out + b) = *reinterpret_cast<const uint32_t *>(&s_out[kv][b]);
+          store4_stream(out + b, *reinterpret_cast<const uint32_t *>(&s_out[kv][b]));
         }
       } else {
         for (int32_t b = threadIdx.x * 2; b < bytes; b += k_threads * 2) {
@@ -291,7 +288,7 @@ void launch_gather(const pool_layout &L, hipStream_t st, const uint8_t *k_pool,
                    const uint16_t *tables, int32_t table_stride, uint8_t *k_out, uint8_t *v_out,
                    int32_t out_tokens) {
   const bool f16 = L.kv_type == EMELK_KV_F16;
-  const int32_t run = f16 ? k_gather_tokens : 4096 / D;
+  const int32_t run = f16 ? k_threads / (D / 8) : 4096 / D;
   const uint64_t units = static_cast<uint64_t>(n_seq) * L.n_head_kv * ((out_tokens - 1) / run + 1);
   constexpr uint64_t cap = 1u << 22;  // workgroups; runs beyond them are taken in turn
   const dim3 grid(static_cast<uint32_t>(units < cap ? units : cap));
@@ -320,20 +317,22 @@ __global__ __launch_bounds__(k_threads) void copy_blocks_kernel(pool_layout L,
   const uint8_t *s = pool + L.region_offset(layer, src, 0);
   uint8_t *d = pool + L.region_offset(layer, dst, 0);
   const uint64_t n16 = L.page_bytes / 16u;
-  // batches of 8 loads issued before their stores keep 8 x 16 B per thread
-  // in flight; the source is read once, so its loads carry the
-  // non-temporal hint (measured 311 vs 337 us for the config-5 compaction,
-  // 218 moves x 32 layers x K,V; non-temporal stores as well: 340 us)
+  // batches of 8 loads issued before their stores keep 8 x 16 B per thread in
+  // flight; the stores carry the non-temporal hint, as the gather's do.  Against
+  // hinted loads and plain stores: 218 moves x 32 layers of 64 KiB pages (1.83
+  // GB) 370 -> 367 us, 40 moves x 32 53.7 -> 50.0, 40 x 8 19.9 -> 13.9 (the pool
+  // in the cache).  16 loads in flight: 357, 51.1, 13.9, but 193 -> 202 for 218
+  // moves of q8_0 pages.
   constexpr int kB = 8;
   uint64_t i = threadIdx.x;
   for (; i + (kB - 1) * k_threads < n16; i += kB * k_threads) {
     uint4_t v[kB];
 #pragma unroll
-    for (int b = 0; b < kB; ++b) v[b] = load16_stream(s + (i + b * k_threads) * 16u);
+    for (int b = 0; b < kB; ++b) v[b] = load16(s + (i + b * k_threads) * 16u);
 #pragma unroll
-    for (int b = 0; b < kB; ++b) store16(d + (i + b * k_threads) * 16u, v[b]);
+    for (int b = 0; b < kB; ++b) store16_stream(d + (i + b * k_threads) * 16u, v[b]);
   }
-  for (; i < n16; i += k_threads) store16(d + i * 16u, load16_stream(s + i * 16u));
+  for (; i < n16; i += k_threads) store16_stream(d + i * 16u, load16(s + i * 16u));
 }
 
 int grid_for(uint64_t work_items) {
