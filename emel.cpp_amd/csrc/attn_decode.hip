@@ -1431,10 +1431,14 @@ __global__ __launch_bounds__(k_combine_threads) void combine_kernel(
     a *= r;
 #pragma unroll
     for (int u = 0; u < CH; ++u) {
-      const float f = s0 + u * R < n ? fast_exp2(mlv[u].x - ms) : 0.0f;
-      l = fmaf(mlv[u].y, f, l);
+      // past n: a repeat of s0, left out by zero values and not by a zero
+      // factor alone, since 0 * inf would be NaN (an f16 pool holds +-inf for
+      // values past 65504)
+      const bool in = s0 + u * R < n;
+      const float f = in ? fast_exp2(mlv[u].x - ms) : 0.0f;
+      l = fmaf(in ? mlv[u].y : 0.0f, f, l);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) a[e] = fmaf(av[u][e], f, a[e]);
+      for (int e = 0; e < 4; ++e) a[e] = fmaf(in ? av[u][e] : 0.0f, f, a[e]);
     }
     mx = mn;
   }

@@ -1129,10 +1129,12 @@ __global__ __launch_bounds__(k_merge_threads) void prefill_merge_kernel(prefill_
     a *= f0;
 #pragma unroll
     for (int u = 0; u < CH; ++u) {
-      const float f = s0 + u < n ? fast_exp2((mlv[u].x - ms) * P.c) : 0.0f;
-      l = fmaf(mlv[u].y, f, l);
+      // past n: a repeat of s0, left out by zero values (0 * inf is NaN)
+      const bool in = s0 + u < n;
+      const float f = in ? fast_exp2((mlv[u].x - ms) * P.c) : 0.0f;
+      l = fmaf(in ? mlv[u].y : 0.0f, f, l);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) a[e] = fmaf(av[u][e], f, a[e]);
+      for (int e = 0; e < 4; ++e) a[e] = fmaf(in ? av[u][e] : 0.0f, f, a[e]);
     }
     mx = mn;
   }
