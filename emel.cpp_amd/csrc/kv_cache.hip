@@ -318,21 +318,23 @@ __global__ __launch_bounds__(k_threads) void copy_blocks_kernel(pool_layout L,
   uint8_t *d = pool + L.region_offset(layer, dst, 0);
   const uint64_t n16 = L.page_bytes / 16u;
   // batches of 8 loads issued before their stores keep 8 x 16 B per thread in
-  // flight; the stores carry the non-temporal hint, as the gather's do.  Against
-  // hinted loads and plain stores: 218 moves x 32 layers of 64 KiB pages (1.83
-  // GB) 370 -> 367 us, 40 moves x 32 53.7 -> 50.0, 40 x 8 19.9 -> 13.9 (the pool
-  // in the cache).  16 loads in flight: 357, 51.1, 13.9, but 193 -> 202 for 218
-  // moves of q8_0 pages.
+  // flight; the source is read once, so its loads carry the non-temporal hint.
+  // The hint on the stores instead costs a first pass over pools that other
+  // kernels just wrote, which is what a compaction is: 218 moves x 32 layers
+  // of 64 KiB pages (1.83 GB) 380 -> 441 us, 40 moves x 32 76 -> 108, 40 x 8
+  // 24 -> 32, 218 x 32 of q8_0 pages 196 -> 243; only copies repeated on a pool
+  // that fits the cache gain (40 x 8: 17.2 -> 13.4).  No hint at all: 405, 101,
+  // 31 and 224 on a first pass.
   constexpr int kB = 8;
   uint64_t i = threadIdx.x;
   for (; i + (kB - 1) * k_threads < n16; i += kB * k_threads) {
     uint4_t v[kB];
 #pragma unroll
-    for (int b = 0; b < kB; ++b) v[b] = load16(s + (i + b * k_threads) * 16u);
+    for (int b = 0; b < kB; ++b) v[b] = load16_stream(s + (i + b * k_threads) * 16u);
 #pragma unroll
-    for (int b = 0; b < kB; ++b) store16_stream(d + (i + b * k_threads) * 16u, v[b]);
+    for (int b = 0; b < kB; ++b) store16(d + (i + b * k_threads) * 16u, v[b]);
   }
-  for (; i < n16; i += k_threads) store16_stream(d + i * 16u, load16(s + i * 16u));
+  for (; i < n16; i += k_threads) store16(d + i * 16u, load16_stream(s + i * 16u));
 }
 
 int grid_for(uint64_t work_items) {
