@@ -682,13 +682,13 @@ def decode_contiguous(g, k_pool, v_pool, layer, q, out, kv_lens, max_kv_len, seq
 _PREFILL_WS = {}
 
 
-def _prefill_workspace(g, n_seq, n_q, table_stride, q, stream):
+def _prefill_workspace(g, n_seq, n_q, table_stride, stream):
     """Scratch for the split keys of one prefill call, or None (unsplit).
 
     It comes from torch's allocator, on the stream the call runs on, so it is
     reused only by work ordered after the call.  A call on another stream than
     torch's current one, one under graph capture (whose replays would outlive
-    the scratch) and one on raw addresses run unsplit."""
+    the scratch) and one that finds no memory for it run unsplit."""
     key = (bytes(g), n_seq, n_q, table_stride)
     need = _PREFILL_WS.get(key)
     if need is None:
@@ -698,13 +698,16 @@ def _prefill_workspace(g, n_seq, n_q, table_stride, q, stream):
         if len(_PREFILL_WS) >= 4096:  # the sizes alone, of as many call shapes
             _PREFILL_WS.clear()
         need = _PREFILL_WS[key] = out.value
-    if need == 0 or not _is_tensor(q):
+    if need == 0:
         return None
     if stream is not None and stream != _current_stream():
         return None
     if torch.cuda.is_current_stream_capturing():
         return None
-    return torch.empty(need, dtype=torch.uint8, device="cuda")
+    try:
+        return torch.empty(need, dtype=torch.uint8, device="cuda")
+    except torch.OutOfMemoryError:  # a full card: the call needs no scratch to run
+        return None
 
 
 def prefill_chunk(g, k_pool, v_pool, layer, q, out, q_start, block_tables, scale, stream=None):
@@ -719,7 +722,7 @@ def prefill_chunk(g, k_pool, v_pool, layer, q, out, q_start, block_tables, scale
     _ints(q_start, "q_start", n_seq)
     _tables(block_tables, n_seq)
     stride = int(block_tables.shape[1])
-    ws = _prefill_workspace(g, n_seq, n_q, stride, q, stream)
+    ws = _prefill_workspace(g, n_seq, n_q, stride, stream)
     _check(lib.emelk_attn_prefill_chunk_ws(ctypes.byref(g), k_pool.data_ptr(), v_pool.data_ptr(),
                                            layer, q.data_ptr(), out.data_ptr(), n_seq, n_q,
                                            q_start.data_ptr(), block_tables.data_ptr(), stride,
