@@ -61,6 +61,16 @@ namespace {
 
 emel_error_type hip_ok(hipError_t e) { return e == hipSuccess ? EMELK_ERR_NONE : EMELK_ERR_BACKEND; }
 
+// The workspace at its largest, or at least at `need` bytes on a full card.
+bool alloc_workspace(emelk_batch_decoder *d, uint64_t most, uint64_t need) {
+  d->ws_bytes = most;
+  if (hipMalloc(&d->d_ws, most) == hipSuccess) return true;
+  (void)hipGetLastError();  // the refusal is dealt with: later calls check their own
+  d->d_ws = nullptr;
+  d->ws_bytes = need;
+  return need < most && hipMalloc(&d->d_ws, need) == hipSuccess;
+}
+
 }  // namespace
 
 extern "C" emel_error_type emelk_batch_decoder_create(const emelk_kv_geometry *g,
@@ -86,8 +96,9 @@ extern "C" emel_error_type emelk_batch_decoder_create(const emelk_kv_geometry *g
   if (emelk_attn_decode_workspace_size(g, max_batch, max_kv_len, &ws) != EMELK_ERR_NONE) {
     return EMELK_ERR_INVALID_REQUEST;
   }
-  // one workspace serves both: a layer call runs either
-  ws = std::max(ws, emelk::prefill_workspace_bound(g, max_kv_len));
+  // one workspace serves both: a layer call runs either.  Decode cannot do
+  // without its part; more than that only lets a prefill split its keys.
+  const uint64_t ws_most = std::max(ws, emelk::prefill_workspace_bound(g, max_kv_len));
   auto *d = new (std::nothrow) emelk_batch_decoder();
   if (d == nullptr) return EMELK_ERR_OUT_OF_MEMORY;
   d->g = *g;
@@ -98,13 +109,12 @@ extern "C" emel_error_type emelk_batch_decoder_create(const emelk_kv_geometry *g
   d->max_batch = max_batch;
   d->max_kv_len = max_kv_len;
   d->stride = stride;
-  d->ws_bytes = ws;
   const size_t tb = static_cast<size_t>(max_batch) * stride * sizeof(uint16_t);
   const size_t ib = static_cast<size_t>(max_batch) * sizeof(int32_t);
   bool ok = hipMalloc(reinterpret_cast<void **>(&d->d_tables), tb) == hipSuccess &&
             hipMalloc(reinterpret_cast<void **>(&d->d_pos), ib) == hipSuccess &&
             hipMalloc(reinterpret_cast<void **>(&d->d_kv_len), ib) == hipSuccess &&
-            hipMalloc(&d->d_ws, ws) == hipSuccess;
+            alloc_workspace(d, ws_most, ws);
   for (auto &s : d->st) {
     ok = ok && hipHostMalloc(reinterpret_cast<void **>(&s.tables), tb, hipHostMallocDefault) == hipSuccess &&
          hipHostMalloc(reinterpret_cast<void **>(&s.pos), ib, hipHostMallocDefault) == hipSuccess &&

@@ -455,7 +455,9 @@ emel_error_type emelk_kv_cache_upload_view(emelk_kv_cache *cache, emelk_kv_actor
  * It uses the actor, the device cache and the rope table it is given (all
  * must outlive it) and allocates its own block-table, position and
  * workspace buffers for up to max_batch sequences of up to max_kv_len
- * tokens.  `stream` must be the stream the cache was created with, so page
+ * tokens.  The workspace is decode's (emelk_attn_decode_workspace_size), or
+ * 64 MiB where steps of several tokens can use more and the device has it.
+ * `stream` must be the stream the cache was created with, so page
  * copies and kernels stay ordered. */
 typedef struct emelk_batch_decoder emelk_batch_decoder;
 emel_error_type emelk_batch_decoder_create(const emelk_kv_geometry *g, emelk_kv_actor *actor,

@@ -1,12 +1,15 @@
 """The scratch a chunked prefill takes to split its keys is a means to speed
 only: a call that cannot have it runs unsplit, as every call did without one."""
 import ctypes
+import os
+import subprocess
 
 import numpy as np
 import pytest
 
 import emelk
 
+ROOT = os.path.normpath(os.path.join(os.path.dirname(__file__), ".."))
 G = (1, 32, 8, 128, 32, 64)
 
 
@@ -31,6 +34,20 @@ def test_no_memory_for_the_scratch_means_none(monkeypatch):
     monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
     assert emelk._prefill_workspace(g, 1, 6, 64, None) is None
     assert asked == [_need(g, 1, 6, 64)] and asked[0] > 0
+
+
+def test_executor_without_memory_for_the_scratch(tmp_path):
+    """The executor is made with the workspace decode needs where there is no
+    room for the prefill's, and refuses only without the former."""
+    exe = str(tmp_path / "batch_decoder_memory")
+    subprocess.run(["g++", "-std=c++20", "-Wall", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
+                    "-I", os.path.join(ROOT, "include"),
+                    "-I", os.path.join(ROOT, "emel.cpp_amd", "csrc"),
+                    os.path.join(ROOT, "tests", "cpp", "batch_decoder_memory.cpp"),
+                    os.path.join(ROOT, "emel.cpp_amd", "csrc", "batch_decoder.cpp"), "-o", exe],
+                   check=True)
+    res = subprocess.run([exe], capture_output=True, text=True, timeout=60)
+    assert res.returncode == 0 and res.stdout.strip() == "ok", res.stdout + res.stderr
 
 
 def _case(device, n_q=6, ctx=1900):
