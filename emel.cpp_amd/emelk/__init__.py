@@ -680,6 +680,7 @@ def decode_contiguous(g, k_pool, v_pool, layer, q, out, kv_lens, max_kv_len, seq
 
 
 _PREFILL_WS = {}
+_CAPTURE_RELAXED = 2  # hipStreamCaptureModeRelaxed
 
 
 def _prefill_workspace(g, n_seq, n_q, table_stride, stream):
@@ -704,10 +705,16 @@ def _prefill_workspace(g, n_seq, n_q, table_stride, stream):
         return None
     if torch.cuda.is_current_stream_capturing():
         return None
+    # A new block is a hipMalloc, which a capture of another thread in global
+    # mode refuses to every thread that has not relaxed its own.
+    mode = ctypes.c_int(_CAPTURE_RELAXED)
+    lib.hipThreadExchangeStreamCaptureMode(ctypes.byref(mode))
     try:
         return torch.empty(need, dtype=torch.uint8, device="cuda")
     except torch.OutOfMemoryError:  # a full card: the call needs no scratch to run
         return None
+    finally:
+        lib.hipThreadExchangeStreamCaptureMode(ctypes.byref(mode))
 
 
 def prefill_chunk(g, k_pool, v_pool, layer, q, out, q_start, block_tables, scale, stream=None):

@@ -95,3 +95,48 @@ def test_prefill_on_a_full_card(device):
         torch.cuda.set_per_process_memory_fraction(1.0)
     torch.cuda.synchronize()
     assert torch.equal(out, whole)
+
+
+@pytest.mark.gpu
+def test_prefill_while_another_thread_captures(device):
+    """Another thread's graph capture in its default (global) mode forbids new
+    device memory to every thread that has not relaxed it; a chunk call beside
+    it runs, split, and the captured graph is what it would be."""
+    import threading
+
+    import torch
+    print("\n[gpu-case] prefill chunk beside another thread's graph capture", flush=True)
+    call, q, _ = _case(device)
+    side, work = torch.cuda.Stream(), torch.cuda.Stream()
+    want, out = torch.full_like(q, float("nan")), torch.full_like(q, float("nan"))
+    x = torch.arange(1000, dtype=torch.float32, device=device)
+    with torch.cuda.stream(work):
+        call(want)
+    torch.cuda.synchronize()
+    begun, done, failed = threading.Event(), threading.Event(), []
+
+    def chunk():
+        begun.wait(60)
+        try:
+            with torch.cuda.stream(work):
+                call(out)
+        except Exception as e:  # noqa: BLE001
+            failed.append(e)
+        done.set()
+
+    t = threading.Thread(target=chunk)
+    t.start()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):  # empties the allocator's cache first
+        y = x * 2.0
+        begun.set()
+        assert done.wait(60)
+        y = y + 1.0
+    t.join()
+    assert not failed, failed
+    for i in range(3):
+        x.fill_(float(i))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, x * 2.0 + 1.0)
+    assert torch.equal(out, want)
