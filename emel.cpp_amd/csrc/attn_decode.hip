@@ -1416,14 +1416,21 @@ __global__ __launch_bounds__(k_combine_threads) void combine_kernel(
     float4_t av[CH];
 #pragma unroll
     for (int u = 0; u < CH; ++u) {
+      // past n: no split, as one without tokens (a repeat of another's sums
+      // times 0 would be NaN where they hold an infinity, which an f16 pool
+      // does for values past 65504)
+      mlv[u] = float2{-INFINITY, 0.0f};
+      av[u] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
       const int32_t sp = s0 + u * R;
-      const uint64_t k = static_cast<uint64_t>(sp < n ? sp : s0) * stride;
-      mlv[u] = *reinterpret_cast<const float2 *>(ml + 2 * k);
-      av[u] = *reinterpret_cast<const float4_t *>(pa + k * D);
+      if (sp < n) {
+        const uint64_t k = static_cast<uint64_t>(sp) * stride;
+        mlv[u] = *reinterpret_cast<const float2 *>(ml + 2 * k);
+        av[u] = *reinterpret_cast<const float4_t *>(pa + k * D);
+      }
     }
     float cm = mlv[0].x;
 #pragma unroll
-    for (int u = 1; u < CH; ++u) cm = fmaxf(cm, mlv[u].x);  // a repeated split changes no max
+    for (int u = 1; u < CH; ++u) cm = fmaxf(cm, mlv[u].x);
     const float mn = fmaxf(mx, cm);
     const float ms = mn == -INFINITY ? 0.0f : mn;
     const float r = fast_exp2(mx - ms);  // 0 on the first batch
@@ -1431,14 +1438,10 @@ __global__ __launch_bounds__(k_combine_threads) void combine_kernel(
     a *= r;
 #pragma unroll
     for (int u = 0; u < CH; ++u) {
-      // past n: a repeat of s0, left out by zero values and not by a zero
-      // factor alone, since 0 * inf would be NaN (an f16 pool holds +-inf for
-      // values past 65504)
-      const bool in = s0 + u * R < n;
-      const float f = in ? fast_exp2(mlv[u].x - ms) : 0.0f;
-      l = fmaf(in ? mlv[u].y : 0.0f, f, l);
+      const float f = fast_exp2(mlv[u].x - ms);
+      l = fmaf(mlv[u].y, f, l);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) a[e] = fmaf(in ? av[u][e] : 0.0f, f, a[e]);
+      for (int e = 0; e < 4; ++e) a[e] = fmaf(av[u][e], f, a[e]);
     }
     mx = mn;
   }

@@ -1115,13 +1115,19 @@ __global__ __launch_bounds__(k_merge_threads) void prefill_merge_kernel(prefill_
     float4_t av[CH];
 #pragma unroll
     for (int u = 0; u < CH; ++u) {
-      const uint64_t s = static_cast<uint64_t>(s0 + u < n ? s0 + u : s0);
-      mlv[u] = *reinterpret_cast<const float2 *>(ml + s * rows_all * 2);
-      av[u] = *reinterpret_cast<const float4_t *>(pa + s * rows_all * D);
+      // past n: no split, as one without keys (a repeat of another's sums times
+      // 0 would be NaN where they hold an infinity)
+      mlv[u] = float2{-INFINITY, 0.0f};
+      av[u] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+      if (s0 + u < n) {
+        const uint64_t s = static_cast<uint64_t>(s0 + u);
+        mlv[u] = *reinterpret_cast<const float2 *>(ml + s * rows_all * 2);
+        av[u] = *reinterpret_cast<const float4_t *>(pa + s * rows_all * D);
+      }
     }
     float cm = mlv[0].x;
 #pragma unroll
-    for (int u = 1; u < CH; ++u) cm = fmaxf(cm, mlv[u].x);  // a repeated split changes no max
+    for (int u = 1; u < CH; ++u) cm = fmaxf(cm, mlv[u].x);
     const float mn = fmaxf(mx, cm);
     const float ms = mn == -INFINITY ? 0.0f : mn;
     const float f0 = fast_exp2((mx - ms) * P.c);  // 0 on the first batch
@@ -1129,12 +1135,10 @@ __global__ __launch_bounds__(k_merge_threads) void prefill_merge_kernel(prefill_
     a *= f0;
 #pragma unroll
     for (int u = 0; u < CH; ++u) {
-      // past n: a repeat of s0, left out by zero values (0 * inf is NaN)
-      const bool in = s0 + u < n;
-      const float f = in ? fast_exp2((mlv[u].x - ms) * P.c) : 0.0f;
-      l = fmaf(in ? mlv[u].y : 0.0f, f, l);
+      const float f = fast_exp2((mlv[u].x - ms) * P.c);
+      l = fmaf(mlv[u].y, f, l);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) a[e] = fmaf(in ? av[u][e] : 0.0f, f, a[e]);
+      for (int e = 0; e < 4; ++e) a[e] = fmaf(av[u][e], f, a[e]);
     }
     mx = mn;
   }
