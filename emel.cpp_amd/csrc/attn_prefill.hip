@@ -71,6 +71,7 @@ struct prefill_params {
   int32_t splits;
   float *part_acc;
   float *part_ml;
+  int32_t whole_keys;  // sequences of at most so many keys stay whole
 };
 
 // Split plan of one query tile: its n_tiles key tiles over at most `splits`
@@ -78,7 +79,7 @@ struct prefill_params {
 // twice that keeps one workgroup, which writes the output itself.  The same
 // in the prefill and in the merge kernel.
 constexpr int k_split_min_tiles = 2;
-__host__ __device__ inline int32_t split_tiles(int32_t n_tiles, int32_t splits) {
+__device__ inline int32_t split_tiles(int32_t n_tiles, int32_t splits) {
   const int32_t most = n_tiles / k_split_min_tiles;
   const int32_t n = splits < most ? splits : (most < 1 ? 1 : most);
   return (n_tiles + n - 1) / n;  // tiles per split; 0 without tiles
@@ -231,7 +232,7 @@ __global__ __launch_bounds__(G_WG * RB * k_wave) void prefill_kernel(prefill_par
   int t_first = 0, n_tiles = all_tiles;
   [[maybe_unused]] bool direct = true;  // the only split of its rows: writes out
   if constexpr (SPLIT) {
-    const int per = split_tiles(all_tiles, P.splits);
+    const int per = total > P.whole_keys ? split_tiles(all_tiles, P.splits) : all_tiles;
     t_first = static_cast<int>(blockIdx.y) * per;
     if (blockIdx.y > 0 && t_first >= all_tiles) return;  // uniform; the merge does not read it
     n_tiles = min(all_tiles, t_first + per);
@@ -1090,15 +1091,16 @@ __global__ __launch_bounds__(k_merge_threads) void prefill_merge_kernel(prefill_
                                                                          int32_t rows_per_tile,
                                                                          int32_t key_tile) {
   constexpr int LPR = D / 4;  // threads of a row
-  const uint64_t rows_all = static_cast<uint64_t>(P.n_seq) * P.n_q * P.L.n_head;
-  const uint64_t row = (static_cast<uint64_t>(blockIdx.x) * k_merge_threads + threadIdx.x) / LPR;
-  if (row >= rows_all) return;
+  // 32-bit: the partials of all splits are at most k_split_max_bytes
+  const uint32_t rows_all = static_cast<uint32_t>(P.n_seq) * P.n_q * P.L.n_head;
+  const uint32_t row = (blockIdx.x * k_merge_threads + threadIdx.x) / LPR;
   const uint32_t d = threadIdx.x % LPR * 4;
-  const uint32_t tok = static_cast<uint32_t>(row / P.L.n_head);  // seq * n_q + r
-  const int32_t seq = static_cast<int32_t>(tok / P.n_q);
-  const int32_t r = static_cast<int32_t>(tok % P.n_q);
-  const int32_t q0 = P.q_start[seq];
-  if (q0 < 0) return;  // zeros, written by the first split
+  const uint32_t tok = row / static_cast<uint32_t>(P.L.n_head);  // seq * n_q + r
+  const int32_t seq = static_cast<int32_t>(tok / static_cast<uint32_t>(P.n_q));
+  const int32_t r = static_cast<int32_t>(tok % static_cast<uint32_t>(P.n_q));
+  const int32_t q0 = row < rows_all ? P.q_start[seq] : -1;
+  // zeros, written by the first split, or a whole sequence
+  if (q0 < 0 || q0 + P.n_q <= P.whole_keys) return;
   const int32_t key_end = q0 + min(P.n_q, (r / rows_per_tile + 1) * rows_per_tile);
   const int32_t n_tiles = (key_end + key_tile - 1) / key_tile;
   const int32_t per = split_tiles(n_tiles, P.splits);
@@ -1120,7 +1122,7 @@ __global__ __launch_bounds__(k_merge_threads) void prefill_merge_kernel(prefill_
       mlv[u] = float2{-INFINITY, 0.0f};
       av[u] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
       if (s0 + u < n) {
-        const uint64_t s = static_cast<uint64_t>(s0 + u);
+        const uint32_t s = static_cast<uint32_t>(s0 + u);
         mlv[u] = *reinterpret_cast<const float2 *>(ml + s * rows_all * 2);
         av[u] = *reinterpret_cast<const float4_t *>(pa + s * rows_all * D);
       }
@@ -1143,7 +1145,7 @@ __global__ __launch_bounds__(k_merge_threads) void prefill_merge_kernel(prefill_
     mx = mn;
   }
   const float inv = l > 0.0f ? 1.0f / l : 0.0f;
-  *reinterpret_cast<float4_t *>(P.out + row * D + d) =
+  *reinterpret_cast<float4_t *>(P.out + static_cast<uint64_t>(row) * D + d) =
       float4_t{a.x * inv, a.y * inv, a.z * inv, a.w * inv};
 }
 
@@ -1187,30 +1189,69 @@ uint64_t partial_bytes(const pool_layout &L, int32_t n_seq, int32_t n_q) {  // o
 // 8/1 heads of 256, 148 -> 40; 512 rows after none, 23.5 us unsplit against
 // 25.7 in four splits, which the estimate leaves unsplit.
 constexpr uint64_t k_split_max_bytes = 64u << 20;
+struct split_cost {
+  int64_t workgroups, cus, tile_ns;
+  int64_t merge_ns;  // of one split's partials
+  // the key tiles and the partials alone; what any split call costs beyond them
+  int64_t work_ns(int64_t tiles, int64_t n) const {
+    return (workgroups * n + cus - 1) / cus * ((tiles + n - 1) / n) * tile_ns +
+           (n == 1 ? 0 : n * merge_ns);
+  }
+  static constexpr int64_t split_ns = 6000;
+};
+split_cost cost_of(const pool_layout &L, const prefill_shape &S, int32_t n_seq, int32_t n_q) {
+  int64_t tile_ns = L.head_dim == 64 ? 1400 : L.head_dim == 128 ? 1900 : L.head_dim == 256 ? 2000 : 3200;
+  if (L.kv_type == EMELK_KV_Q8_0) tile_ns = tile_ns * 21 / 10;
+  return {S.workgroups, device_cu_count(), tile_ns,
+          static_cast<int64_t>(partial_bytes(L, n_seq, n_q)) * 2 / 4200};
+}
+int64_t tiles_of(const prefill_shape &S, int64_t max_keys) {
+  return (max_keys + S.key_tile - 1) / S.key_tile;
+}
 int32_t plan_splits(const pool_layout &L, const prefill_shape &S, int32_t n_seq, int32_t n_q,
                     int64_t max_keys) {
   if (L.head_dim == 512 && L.kv_type == EMELK_KV_Q8_0) return 1;  // row by row
-  const int64_t tiles = (max_keys + S.key_tile - 1) / S.key_tile;
-  const int64_t cus = device_cu_count();
-  int64_t tile_ns = L.head_dim == 64 ? 1400 : L.head_dim == 128 ? 1900 : L.head_dim == 256 ? 2000 : 3200;
-  if (L.kv_type == EMELK_KV_Q8_0) tile_ns = tile_ns * 21 / 10;
+  const split_cost C = cost_of(L, S, n_seq, n_q);
+  const int64_t tiles = tiles_of(S, max_keys);
   const uint64_t one = partial_bytes(L, n_seq, n_q);
-  const int64_t merge_ns = static_cast<int64_t>(one) * 2 / 4200;  // of one split's partials
   int64_t most = tiles / k_split_min_tiles;
-  most = most < cus ? most : cus;
+  most = most < C.cus ? most : C.cus;
   if (static_cast<uint64_t>(most) > k_split_max_bytes / one) {
     most = static_cast<int64_t>(k_split_max_bytes / one);
   }
-  int64_t best = 1, best_ns = (S.workgroups + cus - 1) / cus * tiles * tile_ns;
+  int64_t best = 1, best_ns = C.work_ns(tiles, 1);
   for (int64_t n = 2; n <= most; ++n) {
-    const int64_t ns = (S.workgroups * n + cus - 1) / cus * ((tiles + n - 1) / n) * tile_ns + 6000 +
-                       n * merge_ns;
+    const int64_t ns = C.work_ns(tiles, n) + C.split_ns;
     if (ns < best_ns) {
       best_ns = ns;
       best = n;
     }
   }
   return static_cast<int32_t>(best);
+}
+
+// max_keys is a bound, often the block table's width, and a sequence's keys are
+// known on the device: up to the count returned, the splits do not pay and it
+// stays whole; -1: they do not at max_keys either.  By the estimate above but
+// for a split call's fixed cost, since the merge is launched either way (to
+// within a sixteenth, for few steps).  Through tables of 1000 pages, 32/8 heads
+// of 128, us unsplit / all split / by this rule: 8 x 64 rows after 176 tokens
+// 17.6 / 29.4 / 20.1, after 700 31.9 / 28.7 / 28.4, 2 x 512 after 88 29.2 / 34.9
+// / 32.4, 512 after none 23.2 / 26.5 / 25.9, 4 x 6 after 60 10.2 / 11.3 / 11.0.
+// What is left is the merge launch, which a caller that bounds the plan by its
+// lengths does not have.
+int32_t plan_whole(const pool_layout &L, const prefill_shape &S, int32_t n_seq, int32_t n_q,
+                   int64_t max_keys, int64_t splits) {
+  const split_cost C = cost_of(L, S, n_seq, n_q);
+  const int64_t tiles = tiles_of(S, max_keys);
+  const auto pays = [&](int64_t t) {
+    const int64_t most = t / k_split_min_tiles;
+    return C.work_ns(t, splits < most ? splits : most) < C.work_ns(t, 1);
+  };
+  if (!pays(tiles)) return -1;
+  int64_t t = 2 * k_split_min_tiles;
+  while (t < tiles && !pays(t)) t += 1 + t / 16;
+  return static_cast<int32_t>((t < tiles ? t : tiles) - 1) * S.key_tile;
 }
 
 template <int D, int KT, bool Q8, bool M16, bool SPLIT>
@@ -1311,8 +1352,9 @@ emel_error_type prefill_chunk(const emelk_kv_geometry *g, const void *k_pool, co
   if (splits > 1 && splits > static_cast<int64_t>(workspace_bytes / one)) {
     splits = static_cast<int64_t>(workspace_bytes / one);  // as many as the workspace holds
   }
+  P.whole_keys = splits < 2 ? -1 : plan_whole(L, S, n_seq, n_q, max_keys, splits);
   P.n_seq = n_seq;
-  P.splits = splits < 2 ? 1 : static_cast<int32_t>(splits);
+  P.splits = P.whole_keys < 0 ? 1 : static_cast<int32_t>(splits);
   P.part_acc = static_cast<float *>(workspace);
   P.part_ml = P.part_acc + static_cast<uint64_t>(P.splits) * n_seq * n_q * L.n_head * L.head_dim;
   hipStream_t st = static_cast<hipStream_t>(stream);

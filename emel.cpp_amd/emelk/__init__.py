@@ -717,19 +717,26 @@ def _prefill_workspace(g, n_seq, n_q, table_stride, stream):
         lib.hipThreadExchangeStreamCaptureMode(ctypes.byref(mode))
 
 
-def prefill_chunk(g, k_pool, v_pool, layer, q, out, q_start, block_tables, scale, stream=None):
-    """q/out: float32 [n_seq, n_q, n_head, head_dim]."""
+def prefill_chunk(g, k_pool, v_pool, layer, q, out, q_start, block_tables, scale, stream=None,
+                  max_kv_len=None):
+    """q/out: float32 [n_seq, n_q, n_head, head_dim].  max_kv_len: the tokens of the longest
+    sequence, this chunk included, where the caller knows them; the keys' splits are planned
+    for it and for the block table's width otherwise.  It changes the time of a call whose table
+    is much wider than its sequences, and no result beyond the order of the sums."""
     _pools(g, k_pool, v_pool)
     if not _is_tensor(q) or q.dim() < 2:
         raise TypeError("q: expected a device tensor [n_seq, n_q, ...]")
     n_seq, n_q = int(q.shape[0]), int(q.shape[1])
-    width = g.n_head * g.head_dim
-    _rows(q, "q", n_seq, n_q, width)
-    _rows(out, "out", n_seq, n_q, width)
+    row = g.n_head * g.head_dim
+    _rows(q, "q", n_seq, n_q, row)
+    _rows(out, "out", n_seq, n_q, row)
     _ints(q_start, "q_start", n_seq)
     _tables(block_tables, n_seq)
     stride = int(block_tables.shape[1])
-    ws = _prefill_workspace(g, n_seq, n_q, stride, stream)
+    width = stride
+    if max_kv_len is not None:
+        width = max(1, min(stride, -(-int(max_kv_len) // g.block_tokens)))
+    ws = _prefill_workspace(g, n_seq, n_q, width, stream)
     _check(lib.emelk_attn_prefill_chunk_ws(ctypes.byref(g), k_pool.data_ptr(), v_pool.data_ptr(),
                                            layer, q.data_ptr(), out.data_ptr(), n_seq, n_q,
                                            q_start.data_ptr(), block_tables.data_ptr(), stride,

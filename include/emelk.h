@@ -358,7 +358,12 @@ emel_error_type emelk_attn_prefill_chunk(const emelk_kv_geometry *g, const void 
  * for the same inputs.  emelk_attn_prefill_workspace_size gives the bytes one
  * call can use (0 when it would not split; at most 64 MiB); with a
  * smaller workspace the call runs with fewer splits, and with NULL with none.
- * Calls that overlap need a workspace each.  The reference has no counterpart. */
+ * The plan bounds the sequences by the table's width; those too short for it
+ * to pay run unsplit, at the cost of the merge launch (1 to 3 us).  A caller
+ * that knows its longest sequence avoids that: it passes the size function the
+ * pages of that length as table_stride, and the call no more than the bytes
+ * that gives (NULL for 0).  Calls that overlap need a workspace each.  The
+ * reference has no counterpart. */
 emel_error_type emelk_attn_prefill_workspace_size(const emelk_kv_geometry *g, int32_t n_seq,
                                                   int32_t n_q, int32_t table_stride,
                                                   uint64_t *bytes_out);
