@@ -1,8 +1,8 @@
 """Norm + RoPE + append at the edges of the kernel's launch shapes, bit-exact
-against the oracle: every row-slot count a launch takes (by its token count),
-row counts that leave a wave partly filled, adjacent, halved and partial
-pairings, a norm on q or on k alone, v norm with several v heads per wave, and
-rows and weights that lie 4 bytes off any wider boundary."""
+against the oracle: every row-slot count that a launch of each head size takes
+(by its token count), row counts that leave a wave partly filled, adjacent,
+halved and partial pairings, a norm on q or on k alone, v norm with several v
+heads per wave, and rows and weights that lie 4 bytes off any wider boundary."""
 import numpy as np
 import pytest
 
@@ -26,6 +26,14 @@ CASES = [
     (Q8, 8, 2, 256, 16, HALF, 100, "qk", False, 1, 530),      # partial: through LDS
     (F16, 4, 2, 512, 8, HALF, 512, "qk", False, 1, 1100),
     (Q8, 8, 1, 512, 16, ADJ, 400, "", False, 3, 2),
+    (F16, 8, 1, 64, 16, HALF, 64, "qk", False, 3, 2),
+    # 256 and 512 dims at two and four row slots, which a prompt chunk takes
+    (F16, 8, 1, 256, 16, ADJ, 256, "qk", False, 1, 900),
+    (Q8, 8, 1, 256, 16, HALF, 256, "qk", True, 3, 500),
+    (F16, 8, 1, 256, 12, HALF, 100, "q", False, 1, 1500),
+    (F16, 8, 1, 512, 16, HALF, 512, "qk", True, 1, 1500),
+    (Q8, 8, 1, 512, 8, ADJ, 400, "k", False, 5, 300),
+    (F16, 8, 1, 512, 16, HALF, 300, "qk", False, 1, 1500),
 ]
 
 
