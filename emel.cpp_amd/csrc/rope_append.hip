@@ -129,7 +129,13 @@ __device__ __forceinline__ float v_scale(const float *__restrict__ v, int32_t n,
 // (the reference's order), so the squares go through LDS to one lane per row:
 // RW rows are summed at once, where one lane per wave summing row after row
 // had made it the whole cost.
-template <int D, int NI>
+//
+// NORMS: some norm is asked for; Q8: a q8_0 pool.  Launches without either are
+// kernels of their own, with a third to a half of the registers (31 against 92
+// at head_dim 512, one slot): with the norms in it, 8 x 512 rows of 8/1 heads
+// of 512 took 28.0 us and 11 x 276 22.6, 26.2 and 20.9 without; 64/8 heads of
+// 128 72 and 62.
+template <int D, int NI, bool NORMS, bool Q8>
 __global__ __launch_bounds__(k_waves *k_wave) void rope_append_kernel(rope_append_args A) {
   constexpr int LPR = D / 4 < k_wave ? D / 4 : k_wave;  // lanes of a row
   constexpr int RPI = k_wave / LPR;                     // rows per load instruction
@@ -204,7 +210,7 @@ __global__ __launch_bounds__(k_waves *k_wave) void rope_append_kernel(rope_appen
     __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
     __builtin_amdgcn_wave_barrier();
   };
-  if (row0 < n_qk && (A.q_norm != nullptr || A.k_norm != nullptr)) {  // uniform
+  if (NORMS && row0 < n_qk && (A.q_norm != nullptr || A.k_norm != nullptr)) {  // uniform
     // apply_headwise_rms_norm (detail.hpp:1073-1082)
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
@@ -248,7 +254,7 @@ __global__ __launch_bounds__(k_waves *k_wave) void rope_append_kernel(rope_appen
       }
     }
   }
-  if (A.v_rms != 0 && row0 + RW > n_qk) {  // uniform
+  if (NORMS && A.v_rms != 0 && row0 + RW > n_qk) {  // uniform
     const float rs = v_scale(v_src, L.n_head_kv * D, lane, A.eps);
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
@@ -336,7 +342,6 @@ __global__ __launch_bounds__(k_waves *k_wave) void rope_append_kernel(rope_appen
     }
   }
 
-  const bool q8 = L.kv_type != EMELK_KV_F16;
 #pragma unroll
   for (int i = 0; i < NI; ++i) {
     const int32_t row = row0 + i * RPI + sub;
@@ -349,12 +354,12 @@ __global__ __launch_bounds__(k_waves *k_wave) void rope_append_kernel(rope_appen
       const float4_t y = x[i][c];
       if (row < L.n_head) {
         *reinterpret_cast<float4_u *>(A.q_out + (static_cast<uint64_t>(tok) * L.n_head + row) * D + d) = y;
-      } else if (!q8 && row < n_rows) {
+      } else if (!Q8 && row < n_rows) {
         // store_fp16_rounded_cache (detail.hpp:3050-3055): RNE per value
         *reinterpret_cast<uint2_u *>(region + (static_cast<uint64_t>(slot) * D + d) * 2u) =
             uint2_u{as_u32(pack_half2(y.x, y.y)), as_u32(pack_half2(y.z, y.w))};
       }
-      if (q8 && row0 + RW > L.n_head) {  // uniform
+      if (Q8 && row0 + RW > L.n_head) {  // uniform
         // quantize_row_q8_0_strided (kernel/detail.hpp:804-824) as
         // quantize_block32: a block is 8 lanes, which share its amax
         float amax = 0.0f;
@@ -393,24 +398,41 @@ __global__ __launch_bounds__(k_waves *k_wave) void rope_append_kernel(rope_appen
 // 387 / 340 / 313 / 510 (694 with one thread per 32-value block).  A decode
 // step of 8 tokens takes 4.6 us (5.4 before, q8_0 8.3).  Waves of a workgroup
 // that take one token's next rows instead of the next token's same rows were
-// no faster (29 and 315 us at four slots).
-constexpr int k_max_slots = 4;
+// no faster (29 and 315 us at four slots).  Rows of 256 and 512 dims without
+// norms take two at most: four leave them fewer waves and, at 10 rows a token,
+// two slots in twelve empty (8 x 512 of 8/1 heads of 256 19.6 us with four, 18.6
+// with two).
+constexpr int k_slots_at(int head_dim, bool norms) { return head_dim > 128 && !norms ? 2 : 4; }
 constexpr int64_t k_enough_waves = 4096;
-template <int D, int NI>
-bool launch_rope(const rope_append_args &A, hipStream_t st) {
+template <int D, int NI, bool NORMS>
+bool launch_rope_slots(const rope_append_args &A, hipStream_t st) {
   constexpr int LPR = D / 4 < k_wave ? D / 4 : k_wave;
   constexpr int RW = NI * (k_wave / LPR);
   const int32_t n_rows = A.L.n_head + 2 * A.L.n_head_kv;
   const int64_t tokens = static_cast<int64_t>(A.n_seq) * A.n_tokens;
   const int64_t parts = (n_rows + RW - 1) / RW;
   if constexpr (NI > 1) {
-    if (tokens * parts < k_enough_waves || RW > n_rows) return launch_rope<D, NI / 2>(A, st);
+    if (tokens * parts < k_enough_waves || RW > n_rows) {
+      return launch_rope_slots<D, NI / 2, NORMS>(A, st);
+    }
   }
   const bool lds = A.q_norm != nullptr || A.k_norm != nullptr || A.pairing == k_pairs_general;
+  const uint32_t lds_bytes = lds ? k_waves * RW * (D + 4) * sizeof(float) : 0;
   const dim3 grid(static_cast<uint32_t>((tokens + k_waves - 1) / k_waves), static_cast<uint32_t>(parts));
-  hipLaunchKernelGGL((rope_append_kernel<D, NI>), grid, dim3(k_waves * k_wave),
-                     lds ? k_waves * RW * (D + 4) * sizeof(float) : 0, st, A);
+  const dim3 block(k_waves * k_wave);
+  if (A.L.kv_type == EMELK_KV_F16) {
+    hipLaunchKernelGGL((rope_append_kernel<D, NI, NORMS, false>), grid, block, lds_bytes, st, A);
+  } else {
+    hipLaunchKernelGGL((rope_append_kernel<D, NI, NORMS, true>), grid, block, lds_bytes, st, A);
+  }
   return hipGetLastError() == hipSuccess;
+}
+
+template <int D>
+bool launch_rope(const rope_append_args &A, hipStream_t st) {
+  return A.q_norm != nullptr || A.k_norm != nullptr || A.v_rms != 0
+             ? launch_rope_slots<D, k_slots_at(D, true), true>(A, st)
+             : launch_rope_slots<D, k_slots_at(D, false), false>(A, st);
 }
 
 // Checks a pairing: every pair inside the head and no dim used twice.
@@ -552,9 +574,9 @@ extern "C" emel_error_type emelk_kv_qkv_rope_append(
                   ? emelk::k_pairs_halves
                   : emelk::k_pairs_general;
   hipStream_t st = static_cast<hipStream_t>(stream);
-  const bool ok = L.head_dim == 64    ? emelk::launch_rope<64, emelk::k_max_slots>(A, st)
-                  : L.head_dim == 128 ? emelk::launch_rope<128, emelk::k_max_slots>(A, st)
-                  : L.head_dim == 256 ? emelk::launch_rope<256, emelk::k_max_slots>(A, st)
-                                      : emelk::launch_rope<512, emelk::k_max_slots>(A, st);
+  const bool ok = L.head_dim == 64    ? emelk::launch_rope<64>(A, st)
+                  : L.head_dim == 128 ? emelk::launch_rope<128>(A, st)
+                  : L.head_dim == 256 ? emelk::launch_rope<256>(A, st)
+                                      : emelk::launch_rope<512>(A, st);
   return ok ? EMELK_ERR_NONE : EMELK_ERR_BACKEND;
 }

@@ -34,6 +34,16 @@ CASES = [
     (F16, 8, 1, 512, 16, HALF, 512, "qk", True, 1, 1500),
     (Q8, 8, 1, 512, 8, ADJ, 400, "k", False, 5, 300),
     (F16, 8, 1, 512, 16, HALF, 300, "qk", False, 1, 1500),
+    # no norm at all (kernels of their own), from one slot to the most
+    (F16, 32, 8, 64, 16, HALF, 64, "", False, 2, 700),
+    (F16, 8, 1, 64, 16, ADJ, 64, "", False, 7, 600),
+    (Q8, 16, 8, 128, 16, HALF, 128, "", False, 1, 2049),
+    (F16, 16, 8, 128, 16, HALF, 128, "", False, 3, 1),
+    (F16, 8, 1, 256, 16, HALF, 256, "", False, 1, 900),
+    (Q8, 8, 1, 256, 12, HALF, 100, "", False, 3, 500),
+    (F16, 8, 1, 512, 16, HALF, 512, "", False, 1, 900),
+    (Q8, 4, 2, 512, 8, ADJ, 512, "", False, 1, 1100),
+    (F16, 8, 1, 512, 16, ADJ, 512, "", False, 3, 2),
 ]
 
 
