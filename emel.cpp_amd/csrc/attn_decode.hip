@@ -1507,10 +1507,10 @@ int32_t plan_heads(const pool_layout &L, int32_t n_seq) {
 // measured slower because every split pays its page-list load and merge),
 // each split a whole number of wave tiles with its page list inside the LDS
 // cache.  A long context of few KV heads takes up to k_split_tiles tiles per
-// split (one for each of a workgroup's waves) before it takes more than
-// k_few_splits splits, whose merge would cost more than the idle CUs: one
-// sequence of 4000 tokens, 8/1 heads of 256: 17.0 us with 250 splits, 11.8
-// with 63.
+// split (one for each of a workgroup's 8 waves, two for each of the 4 at
+// head_dim 512) before it takes more than k_few_splits splits, whose merge
+// would cost more than the idle CUs: one sequence of 4000 tokens, 8/1 heads of
+// 256: 17.0 us with 250 splits, 11.8 with 63.
 constexpr int32_t k_few_splits = 32;
 constexpr int32_t k_split_tiles = 8;
 decode_plan plan_decode(const pool_layout &L, int32_t n_seq, int32_t max_kv_len) {

@@ -1,7 +1,7 @@
 // Page-pool kernels: append (f16 and on-the-fly q8_0), block-table gather and
 // batched page copies (copy-on-write tail split, eviction compaction), plus
-// the device KV owner object.  All are HBM-bound byte/integer work: 16-byte
-// coalesced accesses, no LDS, no MFMA.
+// the device KV owner object.  All are HBM-bound byte/integer work on 16-byte
+// coalesced accesses; the q8_0 gather puts its rows together in LDS.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
