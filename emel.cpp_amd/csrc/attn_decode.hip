@@ -1411,7 +1411,8 @@ __global__ __launch_bounds__(k_combine_threads) void combine_kernel(
   const float *pa = part_acc + base * D + d;
   float mx = -INFINITY, l = 0.0f;
   float4_t a = {0.0f, 0.0f, 0.0f, 0.0f};
-  for (int32_t s0 = grp; s0 < n; s0 += R * CH) {
+  // FULL: every split of the batch is there, and its loads need no condition
+  auto batch = [&]<bool FULL>(int32_t s0) {
     float2 mlv[CH];
     float4_t av[CH];
 #pragma unroll
@@ -1422,7 +1423,7 @@ __global__ __launch_bounds__(k_combine_threads) void combine_kernel(
       mlv[u] = float2{-INFINITY, 0.0f};
       av[u] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
       const int32_t sp = s0 + u * R;
-      if (sp < n) {
+      if (FULL || sp < n) {
         const uint64_t k = static_cast<uint64_t>(sp) * stride;
         mlv[u] = *reinterpret_cast<const float2 *>(ml + 2 * k);
         av[u] = *reinterpret_cast<const float4_t *>(pa + k * D);
@@ -1444,7 +1445,10 @@ __global__ __launch_bounds__(k_combine_threads) void combine_kernel(
       for (int e = 0; e < 4; ++e) a[e] = fmaf(av[u][e], f, a[e]);
     }
     mx = mn;
-  }
+  };
+  int32_t s0 = grp;
+  for (; s0 + (CH - 1) * R < n; s0 += R * CH) batch.template operator()<true>(s0);
+  if (s0 < n) batch.template operator()<false>(s0);
   *reinterpret_cast<float4_t *>(&s_acc[grp][d]) = a;
   if (d == 0) s_ml[grp] = float2{mx, l};
   __syncthreads();
