@@ -27,7 +27,7 @@
 //   At the end each wave merges its token groups (halving exchanges) and
 //   writes one partial (m, l, acc[D]) per (sequence, head, split), or the
 //   output itself when a sequence has one split; a second kernel merges the
-//   splits.  For 2 to 64 sequences the splits are balanced over the batch's
+//   splits.  For 2 to 127 sequences the splits are balanced over the batch's
 //   actual lengths.
 //
 // q8_0 pools keep their int8 values exact: biased fp16 (b + 1152) for the
@@ -128,9 +128,11 @@ inline int32_t pow2_shift(int32_t bt) {
   return -1;
 }
 
-// Balanced split plan of a batch of n_seq <= 64 sequences, the same in every
-// wave that computes it: lane i holds sequence i's length, its split count
-// s_i and the index of its first split (exclusive prefix).  Splits are tb
+// Balanced split plan of a batch of n_seq <= k_max_balanced sequences, the same
+// in every wave that computes it: lane i holds the plan of sequence i and, in a
+// batch of more than 64 (W = 2), of sequence i + 64, whose splits follow.  The
+// two are code of their own: with the second half behind a condition, batches of
+// up to 64 took 0.5 to 1.5 us longer.  Splits are tb
 // tiles of `tile` tokens, as few as keep their number within cap (one round of
 // workgroups): tb = ceil(T / (cap - n_seq)) over the batch's T tiles does, as
 // sum s_i <= T / tb + n_seq, and so does most_tiles, at which every sequence is
@@ -149,13 +151,29 @@ __device__ __forceinline__ int32_t wave_scan_incl(int32_t x) {
   return x;
 }
 
+constexpr int32_t k_max_balanced = 2 * k_wave - 1;
+struct seq_plan {
+  int32_t len;
+  int32_t splits;
+  int32_t first;  // index of its first split (exclusive prefix)
+};
+template <int W>
 __device__ __forceinline__ void balanced_splits(const int32_t *__restrict__ kv_lens, int32_t n_seq,
                                                 int32_t cap, int32_t most_tiles, int32_t tile,
-                                                int32_t lane, int32_t &len_i, int32_t &s_i,
-                                                int32_t &excl_i, int32_t &tb) {
-  len_i = lane < n_seq ? kv_lens[lane] : 0;
-  const int32_t t_i = len_i > 0 ? (len_i + tile - 1) / tile : 0;
-  const int32_t incl = wave_scan_incl(t_i);
+                                                int32_t lane, seq_plan (&q)[W], int32_t &tb) {
+  int32_t t[W];
+  int32_t mine = 0;
+#pragma unroll
+  for (int i = 0; i < W; ++i) {
+    const int32_t seq = lane + i * k_wave;
+    q[i].len = seq < n_seq ? kv_lens[seq] : 0;
+  }
+#pragma unroll
+  for (int i = 0; i < W; ++i) {
+    t[i] = q[i].len > 0 ? (q[i].len + tile - 1) / tile : 0;
+    mine += t[i];
+  }
+  const int32_t incl = wave_scan_incl(mine);
   const int32_t T = __builtin_amdgcn_readlane(incl, k_wave - 1);
   tb = cap > n_seq ? (T + (cap - n_seq) - 1) / (cap - n_seq) : most_tiles;
   tb = tb < 1 ? 1 : (tb > most_tiles ? most_tiles : tb);
@@ -166,7 +184,10 @@ __device__ __forceinline__ void balanced_splits(const int32_t *__restrict__ kv_l
   for (int k = 0; k < 3; ++k) {
     const int32_t mid = k == 0 ? lo : lo + (tb - lo) / 2;
     if (lo < tb) {  // uniform
-      const int32_t used = __builtin_amdgcn_readlane(wave_scan_incl((t_i + mid - 1) / mid), k_wave - 1);
+      int32_t n = 0;
+#pragma unroll
+      for (int i = 0; i < W; ++i) n += (t[i] + mid - 1) / mid;
+      const int32_t used = __builtin_amdgcn_readlane(wave_scan_incl(n), k_wave - 1);
       if (used <= cap) {
         tb = mid;
       } else {
@@ -174,8 +195,38 @@ __device__ __forceinline__ void balanced_splits(const int32_t *__restrict__ kv_l
       }
     }
   }
-  s_i = (t_i + tb - 1) / tb;
-  excl_i = wave_scan_incl(s_i) - s_i;
+  int32_t n = 0;
+#pragma unroll
+  for (int i = 0; i < W; ++i) {
+    q[i].splits = (t[i] + tb - 1) / tb;
+    n += q[i].splits;
+  }
+  q[0].first = wave_scan_incl(n) - n;
+  if constexpr (W == 2) q[1].first = q[0].first + q[0].splits;
+}
+
+// The sequence of split w of the plan, the split's index in it, its length and
+// the tiles of a split; false past the last split.  Uniform.
+template <int W>
+__device__ __forceinline__ bool find_split(const int32_t *__restrict__ kv_lens, int32_t n_seq,
+                                           int32_t cap, int32_t most_tiles, int32_t tile,
+                                           int32_t lane, int32_t w, int32_t &seq, int32_t &split,
+                                           int32_t &len, int32_t &tb) {
+  seq_plan q[W];
+  balanced_splits<W>(kv_lens, n_seq, cap, most_tiles, tile, lane, q, tb);
+#pragma unroll
+  for (int i = 0; i < W; ++i) {
+    const uint64_t hit = __builtin_amdgcn_ballot_w64(q[i].splits > 0 && q[i].first <= w &&
+                                                     w < q[i].first + q[i].splits);
+    if (hit != 0) {  // uniform
+      const int32_t src = __builtin_ctzll(hit);
+      seq = src + i * k_wave;
+      split = w - __builtin_amdgcn_readlane(q[i].first, src);
+      len = __builtin_amdgcn_readlane(q[i].len, src);
+      return true;
+    }
+  }
+  return false;
 }
 
 
@@ -786,13 +837,12 @@ __global__ __launch_bounds__(WPB * TS * k_wave) void decode_kernel(decode_params
   uint32_t slot_stride;
   if (P.balanced) {
     const int32_t w = blockIdx.x;
-    int32_t len_i, s_i, excl_i, tb;
-    balanced_splits(P.kv_lens, P.n_seq, P.cap, P.most_tiles, TT, lane, len_i, s_i, excl_i, tb);
-    const uint64_t hit = __builtin_amdgcn_ballot_w64(s_i > 0 && excl_i <= w && w < excl_i + s_i);
-    if (hit == 0) return;  // uniform: more workgroups than splits
-    seq = __builtin_ctzll(hit);
-    split = w - __builtin_amdgcn_readlane(excl_i, seq);
-    len = __builtin_amdgcn_readlane(len_i, seq);
+    int32_t tb;
+    const bool found =
+        P.n_seq <= k_wave
+            ? find_split<1>(P.kv_lens, P.n_seq, P.cap, P.most_tiles, TT, lane, w, seq, split, len, tb)
+            : find_split<2>(P.kv_lens, P.n_seq, P.cap, P.most_tiles, TT, lane, w, seq, split, len, tb);
+    if (!found) return;  // uniform: more workgroups than splits
     tps = tb * TT;
     slot_base = static_cast<uint64_t>(w) * P.L.n_head + kvh * G;
     slot_stride = 1u;
@@ -1372,7 +1422,8 @@ __global__ __launch_bounds__(WPB * TS * k_wave) void decode_kernel(decode_params
 // load of up to R * CH splits is issued before any is used; the groups merge
 // through LDS.
 constexpr int k_combine_threads = 256;
-template <int D, bool BAL>
+// BAL: sequences per lane of the balanced plan, 0 without one.
+template <int D, int BAL>
 __global__ __launch_bounds__(k_combine_threads) void combine_kernel(
     const float *__restrict__ part_acc, const float *__restrict__ part_ml,
     const int32_t *__restrict__ kv_lens, int32_t n_head, int32_t max_splits,
@@ -1391,14 +1442,15 @@ __global__ __launch_bounds__(k_combine_threads) void combine_kernel(
   int32_t n;
   uint64_t base;
   [[maybe_unused]] uint64_t stride = 1u;
-  if constexpr (BAL) {
-    int32_t len_i, s_i, excl_i, tb;
-    balanced_splits(kv_lens, n_seq, cap, most_tiles, tile, threadIdx.x % k_wave, len_i, s_i,
-                    excl_i, tb);
+  if constexpr (BAL > 0) {
+    seq_plan q[BAL];
+    int32_t tb;
+    balanced_splits<BAL>(kv_lens, n_seq, cap, most_tiles, tile, threadIdx.x % k_wave, q, tb);
     // lengths past max_kv_len (outside the contract) could plan more splits
     // than the grid ran: read only slots the grid has
-    const int32_t first = __builtin_amdgcn_readlane(excl_i, seq);
-    n = __builtin_amdgcn_readlane(s_i, seq);
+    const seq_plan own = seq < k_wave ? q[0] : q[BAL - 1];  // uniform
+    const int32_t first = __builtin_amdgcn_readlane(own.first, seq % k_wave);
+    n = __builtin_amdgcn_readlane(own.splits, seq % k_wave);
     n = first >= cap ? 0 : min(n, cap - first);
     base = static_cast<uint64_t>(first) * n_head + row % n_head;
     stride = static_cast<uint64_t>(n_head);
@@ -1503,7 +1555,7 @@ int32_t plan_heads(const pool_layout &L, int32_t n_seq) {
 }
 
 // This is the host plan: the fixed split size, and the bound on the
-// balanced plan the kernels derive on the device for 2 to 64 sequences
+// balanced plan the kernels derive on the device for 2 to 127 sequences
 // (balanced_splits).
 //
 // Split sizing: about one workgroup per CU (a workgroup is 8 waves, which is
@@ -1528,13 +1580,16 @@ decode_plan plan_decode(const pool_layout &L, int32_t n_seq, int32_t max_kv_len)
   int32_t per = (tiles + k_few_splits - 1) / k_few_splits;
   per = per > k_split_tiles ? k_split_tiles : per;
   const int32_t most = (tiles + per - 1) / per;
-  const bool may_balance = n_seq > 1 && n_seq <= k_wave;
-  // No more workgroups than run at once: 24 sequences in 264 took a second
-  // round for the last eight (55 us; 39 in 256).  Rounded up where the balanced
-  // plan's cap keeps them within that, and where one split per sequence would
-  // leave a long sequence of a large batch to a single workgroup.
-  const bool up = may_balance || target / units < 2;
-  int32_t splits = up ? (target + units - 1) / units : target / units;
+  // Balanced, with no more workgroups than run at once (24 sequences in 264 took
+  // a second round for the last eight, 55 us; 39 in 256).  Splits fixed for the
+  // longest sequence fill more than a round for 65 to 127 equal ones when
+  // rounded up, and leave a long one to few workgroups when rounded down: 32/8
+  // heads of 128, up / down / balanced, 100 of 1000 tokens 100 / 72 / 78 us, 100
+  // of 100 to 4000 306 / 230 / 156, one of 8000 among 100 of 100 310 / 440 / 33.
+  // 128 fill the round with two each, and the plan's search would only add to
+  // that (92 us; 98 balanced).
+  const bool may_balance = n_seq > 1 && n_seq <= k_max_balanced;
+  int32_t splits = (target + units - 1) / units;
   splits = splits < 1 ? 1 : (splits > most ? most : splits);
   int32_t tps = ((max_kv_len + splits - 1) / splits + tile - 1) / tile * tile;
   const int32_t max_tps = ((k_max_split_pages - 2) * L.block_tokens) / tile * tile;
@@ -1615,13 +1670,11 @@ template <int D>
 void launch_combine(dim3 grid, hipStream_t st, const decode_params &P, const int32_t *kv_lens,
                     int32_t n_head, int32_t max_splits, int32_t tps, float *out, int32_t n_seq,
                     int32_t tile) {
-  if (P.balanced) {
-    hipLaunchKernelGGL((combine_kernel<D, true>), grid, dim3(k_combine_threads), 0, st, P.part_acc,
-                       P.part_ml, kv_lens, n_head, max_splits, tps, out, n_seq, P.cap, P.most_tiles, tile);
-  } else {
-    hipLaunchKernelGGL((combine_kernel<D, false>), grid, dim3(k_combine_threads), 0, st, P.part_acc,
-                       P.part_ml, kv_lens, n_head, max_splits, tps, out, n_seq, P.cap, P.most_tiles, tile);
-  }
+  const auto kernel = !P.balanced        ? combine_kernel<D, 0>
+                      : n_seq <= k_wave ? combine_kernel<D, 1>
+                                        : combine_kernel<D, 2>;
+  hipLaunchKernelGGL(kernel, grid, dim3(k_combine_threads), 0, st, P.part_acc, P.part_ml, kv_lens,
+                     n_head, max_splits, tps, out, n_seq, P.cap, P.most_tiles, tile);
 }
 
 }  // namespace

@@ -255,7 +255,7 @@ emel_error_type emelk_kv_copy_blocks(const emelk_kv_geometry *g, void *k_pool, v
  * split count rises as the batch shrinks, so the exact need of one call is
  * not monotone in n_seq); emelk_attn_decode_plan reports the host split
  * plan (tokens_per_split, n_splits per sequence) and the exact workspace need
- * of one call with these arguments.  For 2 to 64 sequences the device
+ * of one call with these arguments.  For 2 to 127 sequences the device
  * rebalances the splits over the actual lengths (never more splits than
  * n_seq * n_splits), so the summation order of a sequence depends on the
  * batch's lengths; results are

@@ -1,8 +1,9 @@
 """Decode where several waves of a workgroup walk one KV head in turn (token
 slices) and the split count follows the lengths: lengths around one tile and
-around one tile per wave, one long sequence among short ones, few KV heads,
-every head size, with the step's token stored in the same call, against the
-fp64 ideal on the stored values and the stored bytes."""
+around one tile per wave, one long sequence among short ones, batches of more
+than 64 sequences, few KV heads, every head size, with the step's token stored
+in the same call, against the fp64 ideal on the stored values and the stored
+bytes."""
 import numpy as np
 import pytest
 
@@ -27,6 +28,14 @@ CASES = [
     (256, 2, 4, 16, Q8, [8, 9, 65, 64, 1100]),
     (512, 1, 8, 16, F16, [1300, 5]),
     (512, 1, 2, 32, Q8, [900, 33, 1]),
+    # two sequences per lane in the plan, and the batches on either side
+    (64, 8, 1, 16, F16, [70] * 64),
+    (64, 8, 2, 16, F16, [3000] + [2 + i for i in range(64)]),
+    (64, 8, 1, 16, Q8, [9] * 80 + [1500] + [130] * 19),
+    (128, 1, 8, 32, F16, [40 + 7 * i for i in range(126)] + [2500]),
+    (256, 2, 4, 16, Q8, [1] * 90 + [700, 3]),
+    (64, 16, 2, 16, F16, [300] * 70),                     # more splits than run at once
+    (64, 8, 1, 16, F16, [60] * 127 + [2000]),             # 128: the host plan
 ]
 
 
