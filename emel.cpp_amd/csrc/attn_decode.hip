@@ -1463,20 +1463,21 @@ __global__ __launch_bounds__(k_combine_threads) void combine_kernel(
   const float *pa = part_acc + base * D + d;
   float mx = -INFINITY, l = 0.0f;
   float4_t a = {0.0f, 0.0f, 0.0f, 0.0f};
-  // FULL: every split of the batch is there, and its loads need no condition
-  auto batch = [&]<bool FULL>(int32_t s0) {
+  // The group's splits, CH at a time.  What is left over a whole number of
+  // batches goes first (CH splits of FULL batches need no condition on their
+  // loads), so that the usual few splits run straight through.
+  auto batch = [&]<bool FULL>(int32_t s0, int32_t here) {
     float2 mlv[CH];
     float4_t av[CH];
 #pragma unroll
     for (int u = 0; u < CH; ++u) {
-      // past n: no split, as one without tokens (a repeat of another's sums
-      // times 0 would be NaN where they hold an infinity, which an f16 pool
-      // does for values past 65504)
+      // past the group's splits: none, as one without tokens (a repeat of
+      // another's sums times 0 would be NaN where they hold an infinity, which
+      // an f16 pool does for values past 65504)
       mlv[u] = float2{-INFINITY, 0.0f};
       av[u] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
-      const int32_t sp = s0 + u * R;
-      if (FULL || sp < n) {
-        const uint64_t k = static_cast<uint64_t>(sp) * stride;
+      if (FULL || u < here) {
+        const uint64_t k = static_cast<uint64_t>(s0 + u * R) * stride;
         mlv[u] = *reinterpret_cast<const float2 *>(ml + 2 * k);
         av[u] = *reinterpret_cast<const float4_t *>(pa + k * D);
       }
@@ -1498,9 +1499,10 @@ __global__ __launch_bounds__(k_combine_threads) void combine_kernel(
     }
     mx = mn;
   };
-  int32_t s0 = grp;
-  for (; s0 + (CH - 1) * R < n; s0 += R * CH) batch.template operator()<true>(s0);
-  if (s0 < n) batch.template operator()<false>(s0);
+  const int32_t mine = n > grp ? (n - grp + R - 1) / R : 0;
+  const int32_t left = mine % CH;
+  if (left != 0) batch.template operator()<false>(grp, left);
+  for (int32_t s0 = grp + left * R; s0 < n; s0 += R * CH) batch.template operator()<true>(s0, CH);
   *reinterpret_cast<float4_t *>(&s_acc[grp][d]) = a;
   if (d == 0) s_ml[grp] = float2{mx, l};
   __syncthreads();
