@@ -394,8 +394,9 @@ __global__ __launch_bounds__(k_waves *k_wave) void rope_append_kernel(rope_appen
 // MI355X with 1 / 2 / 4 / 8 slots at most: 8 x 512 tokens of 16/8 heads of 128
 // with q and k norms and halved pairs 38 / 29 / 28 / 42 us (69 with one lane
 // per wave summing row after row; 4.2 TB/s at 28); 64 x 512 of 32/8 heads,
-// adjacent pairs, 376 / 330 / 304 / 476 (444 before; 4.9 TB/s), on a q8_0 pool
-// 387 / 340 / 313 / 510 (694 with one thread per 32-value block).  A decode
+// adjacent pairs, 376 / 330 / 304 / 476 (444 before; 271, 5.4 TB/s, since such
+// launches have no norm in them), on a q8_0 pool 387 / 340 / 313 / 510 (694 with
+// one thread per 32-value block; now 261).  A decode
 // step of 8 tokens takes 4.6 us (5.4 before, q8_0 8.3).  Waves of a workgroup
 // that take one token's next rows instead of the next token's same rows were
 // no faster (29 and 315 us at four slots).  Rows of 256 and 512 dims without

@@ -356,7 +356,8 @@ emel_error_type emelk_attn_prefill_chunk(const emelk_kv_geometry *g, const void 
  * split over workgroups, whose partial results a second launch merges.  Same
  * results as emelk_attn_prefill_chunk up to summation order, and deterministic
  * for the same inputs.  emelk_attn_prefill_workspace_size gives the bytes one
- * call can use (0 when it would not split; at most 64 MiB); with a
+ * call can use (0 when it would not split; at most 64 MiB, which is enough for
+ * every call).  It is no bound for smaller calls, which may use more; with a
  * smaller workspace the call runs with fewer splits, and with NULL with none.
  * The plan bounds the sequences by the table's width; those too short for it
  * to pay run unsplit, at the cost of the merge launch (1 to 3 us).  A caller
